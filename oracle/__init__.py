@@ -45,7 +45,7 @@ def build(force: bool = False) -> None:
     """Compile liboracle.so (and oracle/_ref when the reference tree exists)."""
     if force or not os.path.exists(LIB_PATH):
         subprocess.run(["make", "-s", "-C", HERE, "liboracle.so"], check=True)
-    if os.path.isdir(REFERENCE_ROOT):
+    if os.path.isfile(os.path.join(REFERENCE_ROOT, "adm.c")):
         subprocess.run(["make", "-s", "-C", HERE, "ref"], check=True)
 
 
