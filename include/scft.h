@@ -267,7 +267,9 @@ int scft_batch_time_eval(scft_batch *b, const double *w, int reps,
                          double *ms_per_eval, double *march_ms);
 /* Per size bucket (in the order of scft_batch_tuning): average duration of one persistent march
  * launch over `reps` (HIP events on the launch stream), its algorithmic HBM
- * bytes (q-slabs written and read back plus O(n) I/O) and instance count. */
+ * bytes (the q-slabs it keeps, written and read back, plus O(n) I/O: every slab,
+ * or every fourth in batches whose slab traffic would outlast their steps) and
+ * instance count. */
 int scft_batch_time_buckets(scft_batch *b, const double *w, int reps,
                             int max_buckets, int *n_buckets, double *ms,
                             double *bytes, int *n_items);

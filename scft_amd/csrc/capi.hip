@@ -67,15 +67,21 @@ struct Bucket {
   int wpc = 0;  // workgroups per CU of the persistent grid (0: as many as fit)
   long long slab_stride = 0;  // doubles per workgroup
   long long slab_base = 0;    // this bucket's region in the scratch (doubles)
-  int stream = 0;             // which of the batch's streams launches it
-  double work = 0.0;          // sum of n N over its instances
 };
 
-// rows per lane of a new bucket (implicit Euler keeps ~8 doubles per row in
-// registers, IRK4 ~11: its variants stop at K = 8) and the bucket of n
-// unknowns: shared with the allocation-free entry point (scft_internal.h)
-int default_K(int cap, int stepper) { return bucket_default_K(cap, stepper == SCFT_STEP_IRK4); }
-int cap_for(int n) { return bucket_capacity(n); }
+// One launch of a sweep: a bucket, or (small) all those of up to 512 unknowns.
+struct Launch {
+  int bucket = 0;       // the bucket, or the first of them: its work-queue counter
+  bool small = false;
+  int* d_items = nullptr;  // instance ids, longest expected run first
+  int n_items = 0;
+  int grid = 0;
+  int Nmax = 0;
+  long long slab_stride = 0, slab_base = 0;
+  int stream = 0;       // which of the batch's streams it goes to
+  double work = 0.0;    // sum of n N over its instances
+  double us = 0.0;      // expected run
+};
 
 }  // namespace
 
@@ -90,13 +96,15 @@ struct scft_batch {
   long long total_u = 0, total_x = 0, total_pw = 0, total_h = 0;
   std::string tune_file;
   std::vector<Bucket> buckets;
+  std::vector<Launch> launches;  // of one sweep, longest expected run first
+  int* d_small_items = nullptr;  // the items of a small launch
+  int seg = 1;                   // slabs kept: every one, or every seg-th (march.hip)
   hipStream_t stream = nullptr;  // main stream: copies, resets, the mixer
-  // buckets run concurrently on the main stream plus kSide side streams:
-  // one stream per bucket for the seven buckets of meshes up to 4096 nodes
-  // (a shared stream serialises its buckets: a sweep of 4096 uniform meshes,
-  // m 32-4096, took 13.2-13.7 ms on four streams against 12.5 ms on one
-  // stream each)
-  static constexpr int kSide = 7;
+  // Buckets run concurrently on the main stream plus kSide side streams.  A
+  // process has four hardware queues: more streams share them, and a shared
+  // queue runs its kernels one after the other, whichever the runtime put
+  // there.  With four streams the pairing is ours (size_scratch).
+  static constexpr int kSide = 3;
   hipStream_t side[kSide] = {};
   hipEvent_t fork = nullptr, join[kSide] = {};
   // device state
@@ -129,7 +137,7 @@ struct scft_batch {
   hipGraphExec_t sweep_exec = nullptr;
   AndersonArgs sweep_args;
   int sweep_inner = 1;
-  int top_bucket = -1;  // the non-empty bucket of most work (n N summed)
+  int top_launch = -1;  // the launch of most work (n N summed)
 };
 
 // Forget the cached sweep graph: the bucket launches or mixer buffers it
@@ -151,63 +159,164 @@ static hipError_t launch_eval(const scft_batch* b, int K, int W, const MarchArgs
   return b->stepper == SCFT_STEP_IRK4 ? launch_irk4(K, W, a, grid, s)
                                       : launch_march(K, W, a, grid, s);
 }
-static int eval_max_grid(const scft_batch* b, int K, int W, int half_max) {
-  return b->stepper == SCFT_STEP_IRK4 ? irk4_max_grid(K, W, half_max)
-                                      : march_max_grid(K, W, half_max);
+static int eval_max_grid(const scft_batch* b, int K, int W, int half_max, int seg) {
+  return b->stepper == SCFT_STEP_IRK4 ? irk4_max_grid(K, W, half_max) : march_max_grid(K, W, seg);
 }
-
 // Algorithmic HBM bytes of one evaluation: q-slabs 1..N/2-1 written once and
 // read back once, plus the O(n) inputs/outputs (x, w, phi_t in; phi, r out).
 static double eval_bytes(int n, int N) {
   return 8.0 * n * (2.0 * (N / 2 - 1)) + 40.0 * n;
 }
+// What a launch that keeps every seg-th slab writes and reads back of them,
+// and the O(n) I/O.
+static double slab_bytes(int n, int N, int seg) {
+  return seg == 1 ? eval_bytes(n, N) : 8.0 * n * (2.0 * (N / 2 / seg)) + 40.0 * n;
+}
 
-// Every non-empty bucket owns a scratch region (the buckets of one sweep run
-// concurrently): grid_b workgroups x N_max/2 slabs x 64 W K doubles.
-// Buckets are spread over the main and side streams, largest work first.
+// About how long a workgroup takes over one step of an instance, in
+// microseconds (measured alone, 0.15 at <1, 1> to 0.69 at <8, 8>).
+static double step_us(int K, int W) {
+  return 0.125 + 0.02 * K + (W > 1 ? 0.1 + 0.03 * W : 0.0);
+}
+
+// A persistent grid's expected run: its longest instance, or all of them
+// spread over the workgroups.
+static double run_us(const scft_batch* b, const Bucket& bk, int grid) {
+  double steps = 0.0;
+  for (int k : bk.items) steps += b->desc[k].N;
+  return step_us(bk.K, bk.W) * std::max<double>(bk.Nmax, steps / std::max(1, grid));
+}
+
+// Every launch of a sweep owns a scratch region (they run concurrently): grid
+// workgroups x kept slabs x doubles per slab.
 static int size_scratch(scft_batch* b) {
   drop_sweep_graph(b);
-  long long need = 0;
-  std::vector<std::pair<double, int>> order;
-  for (size_t i = 0; i < b->buckets.size(); i++) {
-    Bucket& bk = b->buckets[i];
+  const bool irk4 = b->stepper == SCFT_STEP_IRK4;
+  auto grid_of = [&](const Bucket& bk, int seg) {
+    const int mg = eval_max_grid(b, bk.K, bk.W, bk.Nmax / 2, seg);
+    // fewer co-resident workgroups per CU can finish a bucket sooner: its
+    // longest instances set the makespan, and they step faster alone
+    const int cap_grid = bk.wpc > 0 ? std::min(mg, bk.wpc * b->cus) : mg;
+    return std::min<int>(static_cast<int>(bk.items.size()), cap_grid);
+  };
+  int filled = 0, small = 0;
+  bool small_ok = !irk4;
+  double longest = 0.0;
+  for (auto& bk : b->buckets) {
     if (bk.items.empty()) continue;
     if (!variant_exists(b, bk.K, bk.W)) {
       snprintf(g_errmsg, sizeof g_errmsg, "no march variant K=%d W=%d", bk.K, bk.W);
       return SCFT_E_ARG;
     }
-    const int P = 64 * bk.W;
-    const int mg = eval_max_grid(b, bk.K, bk.W, bk.Nmax / 2);
-    if (mg < 1) {
+    const int g = grid_of(bk, 1);
+    if (g < 1) {
       snprintf(g_errmsg, sizeof g_errmsg, "march variant K=%d W=%d does not fit a CU", bk.K,
                bk.W);
       return SCFT_E_ARG;
     }
-    // fewer co-resident workgroups per CU can finish a bucket sooner: its
-    // longest instances set the makespan, and they step faster alone
-    const int cap_grid = bk.wpc > 0 ? std::min(mg, bk.wpc * b->cus) : mg;
-    bk.grid = std::max(1, std::min<int>(static_cast<int>(bk.items.size()), cap_grid));
-    bk.slab_stride = static_cast<long long>(std::max(1, bk.Nmax / 2)) * P * bk.K;
+    filled++;
+    if (bk.cap <= 512) {
+      small++;
+      small_ok = small_ok && bk.W == 1 && bk.K == bk.cap / 64 && bk.wpc == 0;
+    }
+    longest = std::max(longest, run_us(b, bk, g));
+  }
+  // Keep every slab while their traffic (at the ~5 TB/s that mixed stores and
+  // loads reach) takes less time than the longest chain of steps; else keep
+  // every MARCH_SEG-th and march 1.375 times as many steps.  Sweeps measured
+  // both ways, all slabs / every fourth: 1024 uniform meshes (0.8 of the
+  // longest chain) 4.5 / 5.1 ms, 1024 graded (1.2) 9.5 / 11.2; 4096 uniform
+  // (2.9) 12.1 / 10.5, 4096 graded (3.0) 28.5 / 25.8.  A single instance
+  // keeps all of them (scft_debug_slabs reads them).
+  const double traffic_us = b->bytes_all / 5.0e6;
+  b->seg = (!irk4 && b->n_inst > 1 && traffic_us > 1.6 * longest) ? MARCH_SEG : 1;
+
+  b->launches.clear();
+  long long need = 0;
+  Launch group;
+  // one launch for the small buckets when there are more launches than
+  // hardware queues (march_small_kernel)
+  const bool merge = small_ok && small >= 2 && filled > 1 + scft_batch::kSide;
+  std::vector<std::pair<double, int>> merged;
+  long long group_need = 0;
+  for (size_t i = 0; i < b->buckets.size(); i++) {
+    Bucket& bk = b->buckets[i];
+    if (bk.items.empty()) continue;
+    const bool in_group = merge && bk.cap <= 512;
+    bk.grid = std::max(1, grid_of(bk, b->seg));
+    const long long kept = std::max(1, bk.Nmax / 2 / b->seg);
+    bk.slab_stride = kept * march_slab_len(bk.K, bk.W, b->seg);
     bk.slab_base = need;
-    need += bk.slab_stride * bk.grid;
     double work = 0.0;
     for (int k : bk.items) work += static_cast<double>(b->desc[k].n) * b->desc[k].N;
-    bk.work = work;
-    order.push_back({work, static_cast<int>(i)});
+    if (in_group) {
+      // (its own launches, in autotune and time_buckets, use the group's region)
+      if (!group.small) group.bucket = static_cast<int>(i);
+      group.small = true;
+      group.Nmax = std::max(group.Nmax, bk.Nmax);
+      group.work += work;
+      group_need = std::max(group_need, bk.slab_stride * bk.grid);
+      for (int k : bk.items) merged.push_back({step_us(bk.K, bk.W) * b->desc[k].N, k});
+      continue;
+    }
+    need += bk.slab_stride * bk.grid;
+    Launch l;
+    l.bucket = static_cast<int>(i);
+    l.d_items = bk.d_items;
+    l.n_items = static_cast<int>(bk.items.size());
+    l.grid = bk.grid;
+    l.Nmax = bk.Nmax;
+    l.slab_stride = bk.slab_stride;
+    l.slab_base = bk.slab_base;
+    l.work = work;
+    l.us = run_us(b, bk, bk.grid);
+    b->launches.push_back(l);
   }
-  std::sort(order.begin(), order.end(), std::greater<std::pair<double, int>>());
-  b->top_bucket = order.empty() ? -1 : order[0].second;
-  // greedy: next bucket onto the least loaded stream
+  if (merge) {
+    std::stable_sort(merged.begin(), merged.end(),
+                     [](const std::pair<double, int>& p, const std::pair<double, int>& q) {
+                       return p.first > q.first;
+                     });
+    std::vector<int> ids;
+    double us = 0.0;
+    for (auto& m : merged) {
+      ids.push_back(m.second);
+      us += m.first;
+    }
+    if (!b->d_small_items) SCFT_TRY(dalloc(&b->d_small_items, static_cast<size_t>(b->n_inst)));
+    HIPCHK(hipMemcpy(b->d_small_items, ids.data(), sizeof(int) * ids.size(),
+                     hipMemcpyHostToDevice));
+    group.d_items = b->d_small_items;
+    group.n_items = static_cast<int>(ids.size());
+    group.grid = std::max(1, std::min(group.n_items, march_small_max_grid(b->seg)));
+    group.slab_stride = std::max<long long>(1, group.Nmax / 2 / b->seg) *
+                        march_slab_len(8, 1, b->seg);
+    // the small buckets are the first ones: their region starts the scratch
+    group.slab_base = 0;
+    group_need = std::max(group_need, group.slab_stride * group.grid);
+    for (auto& l : b->launches) l.slab_base += group_need;
+    for (auto& bk : b->buckets)
+      if (bk.cap > 512) bk.slab_base += group_need;
+    need += group_need;
+    group.us = std::max(merged.front().first, us / group.grid);
+    b->launches.push_back(group);
+  }
+  // longest expected run first, each onto the stream that is free soonest
+  std::stable_sort(b->launches.begin(), b->launches.end(),
+                   [](const Launch& p, const Launch& q) { return p.us > q.us; });
   double load[1 + scft_batch::kSide] = {};
-  for (auto& o : order) {
-    int s = 0;
+  b->top_launch = -1;
+  for (size_t i = 0; i < b->launches.size(); i++) {
+    Launch& l = b->launches[i];
     for (int t = 1; t <= scft_batch::kSide; t++)
-      if (load[t] < load[s]) s = t;
-    b->buckets[o.second].stream = s;
-    load[s] += o.first;
+      if (load[t] < load[l.stream]) l.stream = t;
+    load[l.stream] += l.us;
+    if (b->top_launch < 0 || l.work > b->launches[b->top_launch].work)
+      b->top_launch = static_cast<int>(i);
   }
   if (need > b->slab_doubles) {
     dfree(b->d_slabs);
+    b->slab_doubles = 0;
     SCFT_TRY(dalloc(&b->d_slabs, static_cast<size_t>(need)));
     b->slab_doubles = need;
   }
@@ -253,37 +362,43 @@ static MarchArgs march_args(const scft_batch* b, const Bucket& bk, int bucket_id
   a.slabs = b->d_slabs + bk.slab_base;
   a.slab_stride = bk.slab_stride;
   a.half_max = bk.Nmax / 2;
+  a.seg = b->seg;
   a.items = bk.d_items;
   a.queue = b->d_counters + bucket_idx;
   a.n_items = static_cast<int>(bk.items.size());
   return a;
 }
 
+static hipError_t launch_part(scft_batch* b, const Launch& l, hipStream_t s) {
+  const Bucket& bk = b->buckets[l.bucket];
+  MarchArgs a = march_args(b, bk, l.bucket);
+  a.slabs = b->d_slabs + l.slab_base;
+  a.slab_stride = l.slab_stride;
+  a.half_max = l.Nmax / 2;
+  a.items = l.d_items;
+  a.n_items = l.n_items;
+  return l.small ? launch_march_small(a, l.grid, s) : launch_eval(b, bk.K, bk.W, a, l.grid, s);
+}
+
 // One evaluation sweep of every instance not marked done: counters reset on
-// the main stream, then one persistent launch per non-empty bucket, the
-// buckets spread over the main and side streams (fork/join through events,
-// which stream capture turns into parallel graph branches).  The buckets are
-// launched smallest first, so that their short, latency-bound grids become
-// resident beside the large buckets' persistent grids.  That order matters
-// when buckets share a stream (a sweep of 4096 uniform meshes on four
-// streams: 13.2 ms against 14.0 ms largest first); with a stream per bucket
-// both orders measure 12.5 ms.
+// the main stream, then the persistent launches (one per non-empty bucket, or
+// one for the small ones), spread over the main and side streams (fork/join through events,
+// which stream capture turns into parallel graph branches).  The longest goes
+// first: its workgroups need whole CUs (<8, 8>: every register of one), and
+// what is launched later fills the CUs that are left.  1024 uniform meshes:
+// the top bucket, 3.05 ms alone, took 3.66 ms launched last beside seven
+// streams.
 static hipStream_t stream_of(scft_batch* b, int s) { return s == 0 ? b->stream : b->side[s - 1]; }
 
 static int enqueue_sweep(scft_batch* b) {
   const int nb = static_cast<int>(b->buckets.size());
   HIPCHK(launch_reset(b->d_counters, nb + 1, b->stream));
   bool used[1 + scft_batch::kSide] = {true};
-  for (auto& bk : b->buckets)
-    if (!bk.items.empty()) used[bk.stream] = true;
+  for (auto& l : b->launches) used[l.stream] = true;
   HIPCHK(hipEventRecord(b->fork, b->stream));
   for (int s = 1; s <= scft_batch::kSide; s++)
     if (used[s]) HIPCHK(hipStreamWaitEvent(b->side[s - 1], b->fork, 0));
-  for (int i = 0; i < nb; i++) {
-    const Bucket& bk = b->buckets[i];
-    if (bk.items.empty()) continue;
-    HIPCHK(launch_eval(b, bk.K, bk.W, march_args(b, bk, i), bk.grid, stream_of(b, bk.stream)));
-  }
+  for (auto& l : b->launches) HIPCHK(launch_part(b, l, stream_of(b, l.stream)));
   for (int s = 1; s <= scft_batch::kSide; s++)
     if (used[s]) {
       HIPCHK(hipEventRecord(b->join[s - 1], b->side[s - 1]));
@@ -308,33 +423,28 @@ static int enqueue_solve_sweep(scft_batch* b, const AndersonArgs& a, int inner) 
   const int nb = static_cast<int>(b->buckets.size());
   HIPCHK(launch_reset(b->d_counters, nb + 1, b->stream));
   bool used[1 + scft_batch::kSide] = {true};
-  for (auto& bk : b->buckets)
-    if (!bk.items.empty()) used[bk.stream] = true;
+  for (auto& l : b->launches) used[l.stream] = true;
   HIPCHK(hipEventRecord(b->fork, b->stream));
   for (int s = 1; s <= scft_batch::kSide; s++)
     if (used[s]) HIPCHK(hipStreamWaitEvent(b->side[s - 1], b->fork, 0));
-  for (int i = 0; i < nb; i++) {  // every bucket's first march, smallest first
-    const Bucket& bk = b->buckets[i];
-    if (bk.items.empty()) continue;
-    HIPCHK(launch_eval(b, bk.K, bk.W, march_args(b, bk, i), bk.grid, stream_of(b, bk.stream)));
-  }
+  // every launch's first march, longest first
+  for (auto& l : b->launches) HIPCHK(launch_part(b, l, stream_of(b, l.stream)));
   // then the inner rounds, queued behind every first march (the largest
   // bucket's included) on streams that share a hardware queue
-  for (int i = 0; i < nb; i++) {
-    const Bucket& bk = b->buckets[i];
-    if (bk.items.empty() || inner < 2 || i == b->top_bucket ||
-        3.0 * bk.work > b->buckets[b->top_bucket].work)
+  for (size_t i = 0; i < b->launches.size(); i++) {
+    const Launch& l = b->launches[i];
+    if (inner < 2 || static_cast<int>(i) == b->top_launch ||
+        3.0 * l.work > b->launches[b->top_launch].work)
       continue;
-    const hipStream_t s = stream_of(b, bk.stream);
-    const MarchArgs ma = march_args(b, bk, i);
+    const hipStream_t s = stream_of(b, l.stream);
     AndersonArgs ai = a;
-    ai.order = bk.d_items;
-    ai.n_inst = static_cast<int>(bk.items.size());
+    ai.order = l.d_items;
+    ai.n_inst = l.n_items;
     ai.active = b->d_counters + nb + 1;
     for (int r = 1; r < inner; r++) {
       HIPCHK(launch_anderson(ai, s));
-      HIPCHK(launch_reset(b->d_counters + i, 1, s));  // the bucket's work queue
-      HIPCHK(launch_eval(b, bk.K, bk.W, ma, bk.grid, s));
+      HIPCHK(launch_reset(b->d_counters + l.bucket, 1, s));  // its work queue
+      HIPCHK(launch_part(b, l, s));
     }
   }
   for (int s = 1; s <= scft_batch::kSide; s++)
@@ -430,18 +540,21 @@ extern "C" int scft_batch_create(scft_batch** out, const scft_batch_desc* dsc) {
   for (int cap = 64; cap <= 4096; cap *= 2) {
     Bucket bk;
     bk.cap = cap;
-    bk.K = default_K(cap, b->stepper);
-    bk.W = cap / 64 / bk.K;
     b->buckets.push_back(bk);
   }
   for (int k : order) {
-    const int c = cap_for(b->desc[k].n);
+    const int c = bucket_capacity(b->desc[k].n);
     for (auto& bk : b->buckets)
       if (bk.cap == c) {
         bk.items.push_back(k);
         bk.nmax = std::max(bk.nmax, b->desc[k].n);
         bk.Nmax = std::max(bk.Nmax, b->desc[k].N);
       }
+  }
+  for (auto& bk : b->buckets) {
+    bk.K = bucket_default_K(bk.cap, b->stepper == SCFT_STEP_IRK4,
+                            static_cast<int>(bk.items.size()), b->cus);
+    bk.W = bk.cap / 64 / bk.K;
   }
   read_tune_file(b);
 
@@ -513,6 +626,7 @@ extern "C" int scft_batch_destroy(scft_batch* b) {
   dfree(b->d_ms);
   dfree(b->d_iters);
   dfree(b->d_mix_order);
+  dfree(b->d_small_items);
   if (b->h_active) (void)hipHostFree(b->h_active);
   for (int s = 0; s < scft_batch::kSide; s++) {
     if (b->side[s]) (void)hipStreamSynchronize(b->side[s]);
@@ -627,7 +741,7 @@ extern "C" int scft_batch_time_buckets(scft_batch* b, const double* w, int reps,
     if (c < max_buckets) {
       if (ms) ms[c] = t / reps;
       double by = 0.0;
-      for (int k : bk.items) by += eval_bytes(b->desc[k].n, b->desc[k].N);
+      for (int k : bk.items) by += slab_bytes(b->desc[k].n, b->desc[k].N, b->seg);
       if (bytes) bytes[c] = by;
       if (n_items) n_items[c] = static_cast<int>(bk.items.size());
     }
@@ -712,8 +826,8 @@ extern "C" int scft_batch_tune_placement(scft_batch* b, int tries, int reps) {
 extern "C" int scft_batch_autotune(scft_batch* b, int reps) {
   if (!b) return SCFT_E_STATE;
   if (reps < 1) reps = 1;
-  const int Ks[] = {1, 2, 4, 8, 16};
-  const int Wsz[] = {1, 2, 4, 8, 16};
+  const int Ks[] = {1, 2, 4, 8};
+  const int Wsz[] = {1, 2, 4, 8};
   // current field: leave d_w as is (callers upload first); clear statuses
   HIPCHK(hipMemsetAsync(b->d_status, 0, sizeof(unsigned) * b->n_inst, b->stream));
   hipEvent_t e0, e1;
@@ -729,7 +843,7 @@ extern "C" int scft_batch_autotune(scft_batch* b, int reps) {
       for (int W : Wsz) {
         if (64 * K * W < bk.nmax || 64 * K * W > 2 * bk.cap) continue;
         if (!variant_exists(b, K, W)) continue;
-        const int mg = eval_max_grid(b, K, W, bk.Nmax / 2);
+        const int mg = eval_max_grid(b, K, W, bk.Nmax / 2, b->seg);
         if (mg < 1) continue;
         const int occ = std::max(1, mg / b->cus);
         for (int wpc = 1; wpc <= occ; wpc++) {
@@ -793,7 +907,7 @@ extern "C" int scft_debug_slabs(scft_batch* b, int inst, double* out) {
   const InstDesc& d = b->desc[0];
   for (auto& bk : b->buckets) {
     if (bk.items.empty()) continue;
-    const int P = 64 * bk.W, K = bk.K, half = d.N / 2;
+    const int P = 64 * bk.W, K = bk.K, half = d.N / 2;  // one instance: every slab is kept
     std::vector<double> raw(static_cast<size_t>(half) * P * K);
     HIPCHK(hipMemcpy(raw.data(), b->d_slabs + bk.slab_base, raw.size() * sizeof(double),
                      hipMemcpyDeviceToHost));

@@ -209,5 +209,62 @@ __device__ __forceinline__ void mat_mul_norm(const dd X[4], const dd Y[4], dd R[
 __device__ __forceinline__ dd shfl_up_dd(dd v, int s) {
   return {__shfl_up(v.h, s), __shfl_up(v.l, s)};
 }
+__device__ __forceinline__ dd shfl_down_dd(dd v, int s) {
+  return {__shfl_down(v.h, s), __shfl_down(v.l, s)};
+}
+__device__ __forceinline__ dd dd_neg(dd a) { return {-a.h, -a.l}; }
+// dd times a double
+__device__ __forceinline__ dd dd_mul_d(dd a, double b) {
+#pragma clang fp contract(off)
+  dd p = two_prod(a.h, b);
+  p.l += a.l * b;
+  return quick_two_sum(p.h, p.l);
+}
+// a / b: the leading quotient and one correction with the exact remainder
+__device__ __forceinline__ dd dd_div(dd a, dd b) {
+#pragma clang fp contract(off)
+  const double inv = 1.0 / b.h;
+  const double q1 = a.h * inv;
+  const dd r = dd_add(a, dd_mul_d(b, -q1));
+  return quick_two_sum(q1, r.h * inv);
+}
+// a / b rounded to double
+__device__ __forceinline__ double dd_quot(double a, dd b) {
+#pragma clang fp contract(off)
+  const double inv = 1.0 / b.h;
+  const double q1 = a * inv;
+  const double r = fma(-q1, b.h, a) - q1 * b.l;
+  return q1 + r * inv;
+}
+
+// The power of two that brings the largest of four leading parts into [1, 2)
+// (1 if there is none): ratios of determinants do not see a common scale, and
+// long products neither overflow nor underflow.
+__device__ __forceinline__ double scale4(double a, double b, double c, double d) {
+  const double mx = fmax(fmax(fabs(a), fabs(b)), fmax(fabs(c), fabs(d)));
+  return (mx > 0.0 && isfinite(mx)) ? ldexp(1.0, -ilogb(mx)) : 1.0;
+}
+__device__ __forceinline__ void norm4(dd& a, dd& b, dd& c, dd& d) {
+  const double sc = scale4(a.h, b.h, c.h, d.h);
+  a = dd_scale(a, sc);
+  b = dd_scale(b, sc);
+  c = dd_scale(c, sc);
+  d = dd_scale(d, sc);
+}
+// (r0, r1) <- (r0, r1) M and (c0, c1) <- M (c0, c1), rescaled likewise
+__device__ __forceinline__ void row_times_mat(dd& r0, dd& r1, const dd M[4]) {
+  const dd n0 = dd_add(dd_mul(r0, M[0]), dd_mul(r1, M[2]));
+  const dd n1 = dd_add(dd_mul(r0, M[1]), dd_mul(r1, M[3]));
+  const double sc = scale4(n0.h, n1.h, 0.0, 0.0);
+  r0 = dd_scale(n0, sc);
+  r1 = dd_scale(n1, sc);
+}
+__device__ __forceinline__ void mat_times_col(const dd M[4], dd& c0, dd& c1) {
+  const dd n0 = dd_add(dd_mul(M[0], c0), dd_mul(M[1], c1));
+  const dd n1 = dd_add(dd_mul(M[2], c0), dd_mul(M[3], c1));
+  const double sc = scale4(n0.h, n1.h, 0.0, 0.0);
+  c0 = dd_scale(n0, sc);
+  c1 = dd_scale(n1, sc);
+}
 
 }  // namespace scft

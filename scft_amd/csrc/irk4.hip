@@ -78,7 +78,6 @@ struct cdd {
   dd re, im;
 };
 __device__ __forceinline__ cdd cdd_from(cd a) { return {dd_from(a.re), dd_from(a.im)}; }
-__device__ __forceinline__ dd dd_neg(dd a) { return {-a.h, -a.l}; }
 __device__ __forceinline__ cdd cdd_add(cdd a, cdd b) { return {dd_add(a.re, b.re), dd_add(a.im, b.im)}; }
 __device__ __forceinline__ cdd cdd_mul(cdd a, cdd b) {
   return {dd_add(dd_mul(a.re, b.re), dd_neg(dd_mul(a.im, b.im))),

@@ -8,31 +8,49 @@
 //                 D = A + dt (B + C) and of the right-hand-side operator A from
 //                 the node coordinates and the field (no atomics: a row reads
 //                 its two adjacent elements itself).
-//   2. factor:   the Thomas pivots u_i = b_i - a_i c_{i-1}/u_{i-1} are a
-//                linear-fractional recurrence; each lane multiplies its K
-//                2x2 matrices [[b_i, -a_i c_{i-1}], [1, 0]], a wave-wide
-//                prefix product (plus a fold over waves) gives every lane the
-//                pivot entering its chunk, then the lane finishes its pivots
-//                sequentially.  The solve then reads
-//                    z_i = r'_i - alpha_i z_{i-1},   x_i = z_i - gamma_i x_{i+1}
-//                with alpha = a/u, gamma = c/u and r' = (A q)/u, all kept in
-//                VGPRs for the whole march.
+//   2. factor:   D is tridiagonal, so its inverse G falls off by fixed factors
+//                away from the diagonal: G_ii = 1 / (u_i + v_i - b_i),
+//                G_ij = f_i G_{i-1,j} below it and h_i G_{i+1,j} above it, with
+//                f_i = -a_i / v_i, h_i = -c_i / u_i and u, v the elimination
+//                pivots from above and from below.  The pivots are ratios of
+//                determinants of leading and trailing blocks; a lane takes the
+//                four determinants its chunk needs, and a prefix and a suffix
+//                product of 2x2 matrices over the lanes (and a fold over waves)
+//                give the pivots at its two ends.  All of it in double-double,
+//                once per evaluation (20-40 us).
 //   3. march:    N implicit-Euler steps D q^{j+1} = A q^j (1D_FEM.c:208-228,
-//                step count of DEALII_SCFT/drivescft.cc:130).  Each first-order
-//                recurrence is split into a lane-local pass, a scan of the
+//                step count of DEALII_SCFT/drivescft.cc:130) as q = G (A q): a
+//                recurrence downwards and one upwards that do not wait for each
+//                other.  Each is split into a lane-local pass, a scan of the
 //                lanes' affine maps over the wave (four DPP row levels, then
 //                two cross-row levels: broadcast DPP moves forward, LDS-
 //                crossbar permutes backward; every multiplier is fixed per
 //                instance, so a level costs one FMA per step), a fold over
-//                waves through LDS in one round trip, and a lane-local re-run.
+//                waves through LDS, and the rows from the two inflows.
 //   4. density:  phi_i = sum_j c_j q_j(i) q_{N-j}(i) (drivescft.cc:184-193 with
-//                romint.c's weights, symmetric in j).  Slabs q_1..q_{N/2-1}
-//                stream to HBM (coalesced: element t of lane p at t*P + p,
-//                raw-buffer stores and loads with non-temporal hints); from
-//                step N/2 on each new slab is paired with the stored slab
-//                N-j, loaded a few steps ahead through a register ring.
+//                romint.c's weights, symmetric in j).  Slabs q_0..q_{N/2-1}
+//                stream to HBM (coalesced, raw-buffer stores and loads with
+//                non-temporal hints); from step N/2 on each new slab is paired
+//                with slab N-j.  Either every slab is kept (SEG = 1: loaded a
+//                few steps ahead through a register ring), or every fourth, and
+//                the second half recomputes the others, four at a time into LDS
+//                (SEG = 4).
 //   5. residual: r = phi - phi_t (1D_FEM.c:274-277), ||r||_inf per instance.
 //
+// What bounds it, and what that gave against a two-sweep solve (elimination
+// down, substitution up, every slab kept) on the same variants:
+//   * one instance, or few: the chain of a step.  The two-sweep solve scans
+//     twice and meets twice at a barrier; here once (one exchange through LDS
+//     costs 0.1-0.2 us).  A step of 255 / 1023 / 2047 / 4095 unknowns takes
+//     0.20 / 0.37 / 0.49 / 0.69 us (0.24 / 0.49 / 0.60 / 0.81 before).
+//   * a full chip: HBM.  Stores and loads of all slabs reach ~5.1 TB/s
+//     whatever the variant (640 G node-steps/s), and at that traffic the clock
+//     falls to 1.6 GHz.  With every fourth slab and 1.375 N steps the vector
+//     units bound it (72% busy at 1.9 GHz): 970-1120 G node-steps/s.
+//   * accuracy: the rows of G are computed in double-double and every weight
+//     is positive, so nothing cancels: phi is 10-100 times closer to an
+//     extended-precision march than with pivots rounded to double (m = 4095,
+//     N = 4096, uniform: 5e-14 against 1.4e-11).
 // No MFMA: nothing here is a dense contraction.
 #include "scft_internal.h"
 #include "device_common.h"
@@ -41,14 +59,16 @@ namespace scft {
 
 template <int W>
 struct MarchShared {
-  double Bw[W];     // forward-scan wave totals (per step)
-  double Cw[W];     // backward-scan wave totals (per step)
+  // forward, then backward wave totals (per step, two sets in turn), and a
+  // place for every other lane's write
+  double tot[2][W > 1 ? 2 * W + 64 * W : 1];
   double Aw[W];     // forward wave transfer products (per instance)
   double Gw[W];     // backward wave transfer products (per instance)
-  double cx[W];     // last super-diagonal of each wave (setup)
-  double gx[W];     // last gamma of each wave (setup)
-  double Mx[W][4][2];  // wave products of the pivot matrices, double-double (setup)
+  double cx[W], ax[W];  // last super-, first sub-diagonal of each wave (setup)
+  double hx[W], fx[W];  // last h, first f of each wave (setup)
+  double Mx[W][4][2];  // wave products of the determinant matrices, double-double (setup)
   double red[W];    // norm reduction
+  double cw[6];     // pairing weights by class (per instance)
   unsigned bad[W];
 };
 
@@ -111,10 +131,10 @@ __device__ __forceinline__ Row assemble_row(const double* __restrict__ x,
   return r;
 }
 
-template <int K, int W>
+template <int K, int W, int SEG>
 __device__ void march_one(const MarchArgs& a, const int inst, const unsigned st0,
                           double* __restrict__ slab, MarchShared<W>& sh,
-                          double* __restrict__ pw_lds, const int tid) {
+                          double* __restrict__ seg_lds, const int tid) {
   constexpr int P = 64 * W;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -129,11 +149,19 @@ __device__ void march_one(const MarchArgs& a, const int inst, const unsigned st0
   const int cmat = __builtin_amdgcn_readfirstlane(d.cmat);
   const int u0 = tid * K;
 
-  // pairing weights of this N into LDS (the previous instance's reads of the
-  // table ended at its residual barrier / in program order for one wave)
+  // The pairing weight of step j depends on how often 2 divides j, up to four
+  // times (the five trapezoid levels), except for the last step: six values
+  // in LDS instead of the table of N/2 + 1, which at N = 8192 kept all but
+  // four workgroups off a CU.  (Small N never read the higher classes.)
+  const int half = N >> 1;
+  if (tid < 6) {
+    const int t = (tid == 5) ? half : 1 << tid;
+    sh.cw[tid] = pw[t < half ? t : half];
+  }
   wg_barrier();
-  for (int i = tid; i <= (N >> 1); i += P) pw_lds[i] = pw[i];
-  wg_barrier();
+  auto weight = [&](const int i) __attribute__((always_inline)) {  // of step N/2 + i
+    return sh.cw[(i == half) ? 5 : min(__builtin_ctz(half + i), 4)];
+  };
 
   // ---------------------------------------------------------------- assembly
   double av[K], bv[K], cv[K], ra[K], rc[K];
@@ -148,114 +176,157 @@ __device__ void march_one(const MarchArgs& a, const int inst, const unsigned st0
   }
 
   // ------------------------------------------------------------ factor scan
-  double cprev = __shfl_up(cv[K - 1], 1);
+  // c of the row left of this lane's chunk, a of the row right of it
+  double cprev = __shfl_up(cv[K - 1], 1), anext = __shfl_down(av[0], 1);
   if constexpr (W > 1) {
     sh.cx[wave] = readlane_d(cv[K - 1], 63);
+    sh.ax[wave] = readlane_d(av[0], 0);
     wg_barrier();
     const double cx_prev = (wave > 0) ? sh.cx[wave - 1] : 0.0;
+    const double ax_next = (wave < W - 1) ? sh.ax[wave + 1 < W ? wave + 1 : wave] : 0.0;
     cprev = (lane == 0) ? cx_prev : cprev;
+    anext = (lane == 63) ? ax_next : anext;
   } else {
     cprev = (lane == 0) ? 0.0 : cprev;
+    anext = (lane == 63) ? 0.0 : anext;
   }
-  dd T[4] = {dd_from(1.0), dd_from(0.0), dd_from(0.0), dd_from(1.0)};
+  const dd p_left = two_prod(av[0], cprev);        // couples the chunk to the row before it
+  const dd p_right = two_prod(anext, cv[K - 1]);   // ... and to the row after it
+  // Determinants of the chunk's rows: A of all of them, Cd without the last,
+  // Bd without the first, Dd without both (three-term recurrences in the rows)
+  dd A = dd_from(bv[0]), Cd = dd_from(1.0), Bd = dd_from(1.0), Dd = dd_from(0.0);
+#pragma unroll
+  for (int t = 1; t < K; t++) {
+    const dd np = dd_neg(two_prod(av[t], cv[t - 1]));
+    const dd An = dd_add(dd_mul_d(A, bv[t]), dd_mul(np, Cd));
+    const dd Bn = dd_add(dd_mul_d(Bd, bv[t]), dd_mul(np, Dd));
+    Cd = A;
+    A = An;
+    Dd = Bd;
+    Bd = Bn;
+    if (t % 4 == 3 && t + 1 < K) norm4(A, Cd, Bd, Dd);
+  }
+  norm4(A, Cd, Bd, Dd);
+  // Adjacent chunks combine as a 2x2 product, whichever side's matrix carries
+  // the coupling: the prefix form T = [[A, C], [-p_left B, -p_left D]] gives
+  // the pivot of the last row before a chunk, T00 / T01; the suffix form
+  // R = [[A, -p_right C], [B, -p_right D]] the pivot (from below) of the first
+  // row after it, R00 / R10.
+  // (One after the other, with the scheduler held between them: together
+  // they would double the registers of the setup, which set the occupancy of
+  // the small variants.)
+  dd up = dd_from(1.0), vn = dd_from(1.0);  // no coupling at the two ends: p = 0
   {
-    double cp = cprev;
+    dd T[4] = {A, Cd, dd_neg(dd_mul(p_left, Bd)), dd_neg(dd_mul(p_left, Dd))};
 #pragma unroll
-    for (int t = 0; t < K; t++) {
-      const dd Mt[4] = {dd_from(bv[t]), two_prod(-av[t], cp), dd_from(1.0), dd_from(0.0)};
-      mat_mul_norm(Mt, T, T);
-      cp = cv[t];
+    for (int lev = 0; lev < 6; lev++) {
+      const int s = 1 << lev;
+      dd Tp[4];
+#pragma unroll
+      for (int e = 0; e < 4; e++) Tp[e] = shfl_up_dd(T[e], s);
+      if (lane >= s) mat_mul_norm(Tp, T, T);
     }
-  }
+    dd pr0 = dd_from(1.0), pr1 = dd_from(0.0);  // row 0 of the product before this wave
+    if constexpr (W > 1) {
 #pragma unroll
-  for (int dd_ = 0; dd_ < 6; dd_++) {
-    const int s = 1 << dd_;
-    dd Tp[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) Tp[e] = shfl_up_dd(T[e], s);
-    if (lane >= s) mat_mul_norm(T, Tp, T);
-  }
-  dd E[4];
-#pragma unroll
-  for (int e = 0; e < 4; e++) E[e] = shfl_up_dd(T[e], 1);
-  dd Pre[4] = {dd_from(1.0), dd_from(0.0), dd_from(0.0), dd_from(1.0)};
-  if constexpr (W > 1) {
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      sh.Mx[wave][e][0] = readlane_d(T[e].h, 63);
-      sh.Mx[wave][e][1] = readlane_d(T[e].l, 63);
+      for (int e = 0; e < 4; e++) {
+        sh.Mx[wave][e][0] = readlane_d(T[e].h, 63);
+        sh.Mx[wave][e][1] = readlane_d(T[e].l, 63);
+      }
+      wg_barrier();
+      for (int v = 0; v < wave; v++) {
+        const dd Mv[4] = {{sh.Mx[v][0][0], sh.Mx[v][0][1]}, {sh.Mx[v][1][0], sh.Mx[v][1][1]},
+                          {sh.Mx[v][2][0], sh.Mx[v][2][1]}, {sh.Mx[v][3][0], sh.Mx[v][3][1]}};
+        row_times_mat(pr0, pr1, Mv);
+      }
+      wg_barrier();  // Mx is written again below
     }
-    wg_barrier();
-    for (int v = 0; v < wave; v++) {
-      const dd Mv[4] = {{sh.Mx[v][0][0], sh.Mx[v][0][1]}, {sh.Mx[v][1][0], sh.Mx[v][1][1]},
-                        {sh.Mx[v][2][0], sh.Mx[v][2][1]}, {sh.Mx[v][3][0], sh.Mx[v][3][1]}};
-      mat_mul_norm(Mv, Pre, Pre);
-    }
-  }
-  if (lane > 0) {
-    mat_mul_norm(E, Pre, E);
-  } else {
 #pragma unroll
-    for (int e = 0; e < 4; e++) E[e] = Pre[e];
+    for (int e = 0; e < 4; e++) T[e] = shfl_up_dd(T[e], 1);
+    if (lane > 0) row_times_mat(pr0, pr1, T);
+    if (tid > 0) up = dd_div(pr0, pr1);
   }
-  // pivot of the row just before this lane's chunk (unused for tid 0: a = 0)
-  double up = (tid > 0) ? dd_div_to_double(E[0], E[2]) : 1.0;
+  __builtin_amdgcn_sched_barrier(0);
+  {
+    dd R[4] = {A, dd_neg(dd_mul(p_right, Cd)), Bd, dd_neg(dd_mul(p_right, Dd))};
+#pragma unroll
+    for (int lev = 0; lev < 6; lev++) {
+      const int s = 1 << lev;
+      dd Rn[4];
+#pragma unroll
+      for (int e = 0; e < 4; e++) Rn[e] = shfl_down_dd(R[e], s);
+      if (lane + s < 64) mat_mul_norm(R, Rn, R);
+    }
+    dd sc0 = dd_from(1.0), sc1 = dd_from(0.0);  // column 0 of the product after this wave
+    if constexpr (W > 1) {
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        sh.Mx[wave][e][0] = readlane_d(R[e].h, 0);
+        sh.Mx[wave][e][1] = readlane_d(R[e].l, 0);
+      }
+      wg_barrier();
+      for (int v = W - 1; v > wave; v--) {
+        const dd Mv[4] = {{sh.Mx[v][0][0], sh.Mx[v][0][1]}, {sh.Mx[v][1][0], sh.Mx[v][1][1]},
+                          {sh.Mx[v][2][0], sh.Mx[v][2][1]}, {sh.Mx[v][3][0], sh.Mx[v][3][1]}};
+        mat_times_col(Mv, sc0, sc1);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) R[e] = shfl_down_dd(R[e], 1);
+    if (lane < 63) mat_times_col(R, sc0, sc1);
+    if (tid < P - 1) vn = dd_div(sc0, sc1);
+  }
+  __builtin_amdgcn_sched_barrier(0);
 
+  // Rows of the inverse (f, h and G_ii of the header).  The pivots stay in
+  // double-double through the chunk: u_i + v_i - b_i cancels when the columns
+  // fall off slowly, and an error of f shared by like rows is multiplied by
+  // the fall-off length and by N.
   unsigned bad = 0;
-  double al[K], ga[K];
+  double f[K], h[K], rd[K];
   {
-#pragma clang fp contract(off)
-    double cp = cprev;
+    dd sl[K];  // u_t - b_t
 #pragma unroll
     for (int t = 0; t < K; t++) {
-      // Thomas order: l = a / u_prev, u = b - l c_prev
-      const double l = (av[t] != 0.0) ? av[t] / up : 0.0;
-      const double uu = bv[t] - l * cp;
-      if (!(uu > 0.0) || !isfinite(uu)) bad |= ST_PIVOT;
-      const double inv = 1.0 / uu;
-      al[t] = av[t] * inv;
-      ga[t] = cv[t] * inv;
-      ra[t] *= inv;
-      rc[t] *= inv;
-      cp = cv[t];
-      up = uu;
+      const dd p = (t == 0) ? p_left : two_prod(av[t], cv[t > 0 ? t - 1 : 0]);
+      sl[t] = dd_neg(dd_div(p, up));
+      up = dd_add(dd_from(bv[t]), sl[t]);
+      if (!(up.h > 0.0) || !isfinite(up.h)) bad |= ST_PIVOT;
+      h[t] = -dd_quot(cv[t], up);
+    }
+#pragma unroll
+    for (int t = K - 1; t >= 0; t--) {
+      const dd p = (t == K - 1) ? p_right : two_prod(av[t + 1 < K ? t + 1 : 0], cv[t]);
+      vn = dd_add(dd_from(bv[t]), dd_neg(dd_div(p, vn)));
+      f[t] = -dd_quot(av[t], vn);
+      const dd gi = dd_add(sl[t], vn);
+      ra[t] = dd_quot(ra[t], gi);
+      rc[t] = dd_quot(rc[t], gi);
+      rd[t] = 2.0 * (ra[t] + rc[t]);
     }
   }
 
   // -------------------------------------------- scan constants of the march
-  // Each lane's chunk is an affine map: forward z_out = Af z_in + B, backward
-  // x_first = Gb x_next + C, with Af = prod(-alpha), Gb = prod(-gamma) fixed
-  // for the instance.  The per-step scans combine these maps over the wave:
-  // a Hillis-Steele scan inside each 16-lane row (DPP row_shr / row_shl by
-  // 1, 2, 4, 8), then two row-to-row levels (forward: DPP row_bcast:15 and
+  // A lane's chunk is an affine map in each direction: F leaves it as
+  // Af F_in + B, Y leaves it (upwards) as Gb Y_in + C, with Af = prod f and
+  // Gb = prod h fixed for the instance.  The two scans of a step run side by
+  // side: a Hillis-Steele scan inside each 16-lane row (DPP row_shr / row_shl
+  // by 1, 2, 4, 8), then two row-to-row levels (forward: DPP row_bcast:15 and
   // row_bcast:31; backward: ds_bpermute from the first lane of the next
-  // rows), then (several waves) a fold over wave totals in LDS.  All
-  // multipliers are precomputed here; a step costs one FMA per level.
+  // rows), then (several waves) one fold over the wave totals of both in
+  // LDS.  All multipliers are precomputed here; a step costs one FMA per level.
   const int rl = lane & 15;   // lane within its row
   const int row = lane >> 4;  // row within the wave
-  double Af = 1.0, Gb = 1.0;
+  // Pf_t = f_0 .. f_t and Ph_t = h_t .. h_{K-1}: what the inflows add to row t
+  double Pf[K], Ph[K];
+  Pf[0] = f[0];
+  Ph[K - 1] = h[K - 1];
 #pragma unroll
-  for (int t = 0; t < K; t++) {
-    Af *= -al[t];
-    Gb *= -ga[t];
+  for (int t = 1; t < K; t++) {
+    Pf[t] = Pf[t - 1] * f[t];
+    Ph[K - 1 - t] = Ph[K - t] * h[K - 1 - t];
   }
-  // Within the chunk, z_t = zloc_t + Pf[t] zin with zloc the local pass from
-  // zin = 0 and Pf[t] = prod_{s <= t} (-alpha_s); so the lane's backward offset
-  // (the local backward pass over z) is C0 + Sz zin, C0 the local backward
-  // pass over zloc and Sz = sum_t prod_{s < t} (-gamma_s) Pf[t].  C0 needs no
-  // zin: it runs while the forward scan is in flight, and the final forward
-  // pass leaves the critical path.
-  double Pf[K], Sz = 0.0;
-  {
-    double p = 1.0, g = 1.0;
-#pragma unroll
-    for (int t = 0; t < K; t++) {
-      p *= -al[t];
-      Pf[t] = p;
-      Sz = fma(g, p, Sz);
-      g *= -ga[t];
-    }
-  }
+  double Af = Pf[K - 1], Gb = Ph[0];
   double mf[4], mb[4];
   {
     double Ap, Gp;
@@ -306,7 +377,8 @@ __device__ void march_one(const MarchArgs& a, const int inst, const unsigned st0
   const int srcA = ((row + 1) & 3) * 64;  // byte address of lane 16 (row + 1)
   const int srcB = 32 * 4;
   const double Gsuf_p1 = ((rl < 15) ? Gshift : 1.0) * Gafter;
-  double gl = __shfl_up(ga[K - 1], 1);  // gamma of the row left of me
+  // h of the row left of the chunk, f of the row right of it
+  double hl = __shfl_up(h[K - 1], 1), fr = __shfl_down(f[0], 1);
   // Fold multipliers.  The forward carry into this wave from the waves before
   // it is Z = sum_{v < wave} fz[v] Bw[v] with fz[v] = prod_{v < u < wave} Aw[u];
   // the backward carry from the waves after it is X = sum_{v > wave} fx[v] Cw[v]
@@ -316,11 +388,14 @@ __device__ void march_one(const MarchArgs& a, const int inst, const unsigned st0
   [[maybe_unused]] double fz[W], fx[W];
   if constexpr (W > 1) {
     sh.Aw[wave] = Arow0 * Arow1 * Arow2 * Arow3;
-    sh.gx[wave] = readlane_d(ga[K - 1], 63);
+    sh.hx[wave] = readlane_d(h[K - 1], 63);
+    sh.fx[wave] = readlane_d(f[0], 0);
     sh.Gw[wave] = Grow0 * Grow1 * Grow2 * Grow3;
     wg_barrier();
-    const double gx_prev = (wave > 0) ? sh.gx[wave - 1] : 0.0;
-    gl = (lane == 0) ? gx_prev : gl;
+    const double hx_prev = (wave > 0) ? sh.hx[wave - 1] : 0.0;
+    const double fx_next = (wave < W - 1) ? sh.fx[wave + 1 < W ? wave + 1 : wave] : 0.0;
+    hl = (lane == 0) ? hx_prev : hl;
+    fr = (lane == 63) ? fx_next : fr;
     double p = 1.0;
 #pragma unroll
     for (int v = W - 1; v >= 0; v--) {
@@ -334,7 +409,8 @@ __device__ void march_one(const MarchArgs& a, const int inst, const unsigned st0
       p = (v > wave) ? p * sh.Gw[v] : p;
     }
   } else {
-    gl = (lane == 0) ? 0.0 : gl;
+    hl = (lane == 0) ? 0.0 : hl;
+    fr = (lane == 63) ? 0.0 : fr;
   }
 
   // ------------------------------------------------------------------ march
@@ -346,142 +422,249 @@ __device__ void march_one(const MarchArgs& a, const int inst, const unsigned st0
   }
   double ql = (u0 - 1 >= 0 && u0 - 1 < n) ? 1.0 : 0.0;
   double qr = (u0 + K < n) ? 1.0 : 0.0;
-  const int half = N >> 1;
 
-  // One implicit-Euler step q <- D^{-1} (A q) for the whole instance; ql / qr
+  // One implicit-Euler step q <- G (A q) for the whole instance: with r the
+  // right-hand side scaled by G_ii (ra, rd, rc),
+  //   F_i = r_i + f_i F_{i-1},  Y_i = r_i + h_i Y_{i+1},  q_i = F_i + h_i Y_{i+1},
+  // two recurrences that do not wait for each other, so the lane-local
+  // passes, the scans and the fold over waves (one barrier) overlap; ql / qr
   // become the new values of the unknowns left of q[0] and right of q[K-1].
-  auto advance = [&]() __attribute__((always_inline)) {
-    double rp[K];
+  // How the inflows reach the rows: with the products Pf, Ph (KEEP_P) two
+  // independent FMAs per row after them, which is the shorter chain; without,
+  // the passes run again (the same FMAs, one after the other), which saves 4 K
+  // registers.
+  constexpr bool KEEP_P = SEG == 1 && W < 8;
+  int par = 0;
+  [[maybe_unused]] const int tot_at = (lane == 0) ? W + wave : (lane == 63) ? wave : 2 * W + tid;
+  auto advance = [&](double (&q)[K], double& ql, double& qr) __attribute__((always_inline)) {
+    double r[K];
 #pragma unroll
     for (int t = 0; t < K; t++) {
       const double qm = (t == 0) ? ql : q[t - 1];
       const double qp = (t == K - 1) ? qr : q[t + 1];
-      rp[t] = ra[t] * (qm + 2.0 * q[t]) + rc[t] * (2.0 * q[t] + qp);
+      r[t] = fma(ra[t], qm, fma(rc[t], qp, rd[t] * q[t]));
     }
-    // forward recurrence z_i = r'_i - alpha_i z_{i-1}: the local pass from 0
-    // (zloc kept in rp), and the local backward pass over it
-    double B = 0.0;
+    // local passes from zero inflow: what the chunk adds to its outflows
+    double B = r[0], Cc = r[K - 1];
+    double F0[K], Y0[K];  // (KEEP_P only)
+    F0[0] = B;
+    Y0[K - 1] = Cc;
 #pragma unroll
-    for (int t = 0; t < K; t++) {
-      B = rp[t] - al[t] * B;
-      rp[t] = B;
+    for (int t = 1; t < K; t++) {
+      B = fma(f[t], B, r[t]);
+      Cc = fma(h[K - 1 - t], Cc, r[K - 1 - t]);
+      F0[t] = B;
+      Y0[K - 1 - t] = Cc;
     }
-    double C0 = 0.0;
+    if constexpr (KEEP_P) {  // the chunk's own part of its rows, ready before the inflows are
 #pragma unroll
-    for (int t = K - 1; t >= 0; t--) C0 = rp[t] - ga[t] * C0;
+      for (int t = 0; t + 1 < K; t++) F0[t] = fma(h[t], Y0[t + 1], F0[t]);
+    }
+    const double Bk = B, Ck = Cc;
     B = fma(mf[0], row_shr<1>(B), B);
+    Cc = fma(mb[0], row_shl<1>(Cc), Cc);
     B = fma(mf[1], row_shr<2>(B), B);
+    Cc = fma(mb[1], row_shl<2>(Cc), Cc);
     B = fma(mf[2], row_shr<4>(B), B);
+    Cc = fma(mb[2], row_shl<4>(Cc), Cc);
     B = fma(mf[3], row_shr<8>(B), B);
-    // rows to the whole wave: broadcast levels instead of readlane carries
+    Cc = fma(mb[3], row_shl<8>(Cc), Cc);
+    // carries into rows 0..2 of the backward scan: the suffix from the first
+    // lane of the row after; rows to the whole wave forward: broadcast levels
+    Cc = fma(mbA, bpermute_d(srcA, Cc), Cc);
     B = fma(mf5, row_bcast15(B), B);
+    Cc = fma(mbB, bpermute_d(srcB, Cc), Cc);
     B = fma(mf6, row_bcast31(B), B);
-    // B is now the wave-inclusive prefix; this lane's input is lane - 1's
-    double zin = wave_shr1(B);
+    // wave-inclusive now: this lane's inflows are lane - 1's and lane + 1's
+    double Fin = wave_shr1(B), Yin = wave_shl1(Cc);
     if constexpr (W > 1) {
-      sh.Bw[wave] = readlane_d(B, 63);
+      // two sets of slots in turn: a wave writes the next step's set while a
+      // slower one still reads this step's, and the barrier in between keeps
+      // any wave from being two steps ahead
+      // (lane 63 writes the forward total, lane 0 the backward one, the other
+      // lanes a place of their own: a branch around the write costs 50 ns)
+      sh.tot[par][tot_at] = (lane == 0) ? Cc : B;
       wg_barrier();
-      double Z0 = 0.0, Z1 = 0.0;
+      double Z0 = 0.0, Z1 = 0.0, X0 = 0.0, X1 = 0.0;
 #pragma unroll
       for (int v = 0; v + 1 < W; v += 2) {
-        Z0 = fma(fz[v], sh.Bw[v], Z0);
-        if (v + 2 < W) Z1 = fma(fz[v + 1], sh.Bw[v + 1], Z1);
+        Z0 = fma(fz[v], sh.tot[par][v], Z0);
+        if (v + 2 < W) Z1 = fma(fz[v + 1], sh.tot[par][v + 1], Z1);
+        X0 = fma(fx[v + 1], sh.tot[par][W + v + 1], X0);
+        if (v + 2 < W) X1 = fma(fx[v + 2], sh.tot[par][W + v + 2], X1);
       }
-      zin = fma(Apre_m1, Z0 + Z1, zin);
+      Fin = fma(Apre_m1, Z0 + Z1, Fin);
+      Yin = fma(Gsuf_p1, X0 + X1, Yin);
+      par ^= 1;
     }
-    // backward recurrence x_i = z_i - gamma_i x_{i+1}: this lane's offset
-    double Cc = fma(Sz, zin, C0);
-    Cc = fma(mb[0], row_shl<1>(Cc), Cc);
-    Cc = fma(mb[1], row_shl<2>(Cc), Cc);
-    Cc = fma(mb[2], row_shl<4>(Cc), Cc);
-    Cc = fma(mb[3], row_shl<8>(Cc), Cc);
-    // carries into rows 0..2: the suffix from the first lane of the row after
-    Cc = fma(mbA, bpermute_d(srcA, Cc), Cc);
-    Cc = fma(mbB, bpermute_d(srcB, Cc), Cc);
-    // Cc is now the wave-inclusive suffix; this lane's input is lane + 1's
-    double xin = wave_shl1(Cc);
-    if constexpr (W > 1) {
-      sh.Cw[wave] = readlane_d(Cc, 0);
-      wg_barrier();
-      double X0 = 0.0, X1 = 0.0;
+    if constexpr (KEEP_P) {
+      ql = fma(hl, fma(Ph[0], Yin, Ck), Fin);
+      qr = fma(fr, fma(Pf[K - 1], Fin, Bk), Yin);
 #pragma unroll
-      for (int v = 1; v < W; v += 2) {
-        X0 = fma(fx[v], sh.Cw[v], X0);
-        if (v + 1 < W) X1 = fma(fx[v + 1], sh.Cw[v + 1], X1);
-      }
-      xin = fma(Gsuf_p1, X0 + X1, xin);
-    }
-    {
-      double xx = xin;
+      for (int t = 0; t < K; t++) q[t] = fma(Pf[t], Fin, fma(Ph[t], Yin, F0[t]));
+    } else {
+      // the passes again from the true inflows
+      double Y = Yin, F = Fin;
 #pragma unroll
       for (int t = K - 1; t >= 0; t--) {
-        xx = fma(Pf[t], zin, rp[t]) - ga[t] * xx;  // z_t - gamma_t x_{t+1}
-        q[t] = xx;
+        q[t] = Y;
+        Y = fma(h[t], Y, r[t]);
       }
+#pragma unroll
+      for (int t = 0; t < K; t++) {
+        F = fma(f[t], F, r[t]);
+        q[t] = fma(h[t], q[t], F);
+      }
+      ql = fma(hl, Y, Fin);
+      qr = fma(fr, F, Yin);
     }
-    ql = zin - gl * q[0];
-    qr = xin;
   };
 
-  // Slab s (q after step s, s = 0 .. N/2 - 1; slab 0 is the initial
-  // condition) starts at s * P * K; within it row t of lane tid sits at
-  // (t / 2) * 2P + 2 tid + t % 2 (K >= 2: 16 bytes per lane and access) or at
-  // tid (K = 1).  Lanes whose rows are all
-  // padding (u0 >= n) store nothing (one exec mask for the whole loop) and
-  // load from lane 0's address, so a wave's dead lanes share one cache line;
-  // what they load only ever multiplies their q = 0.  The region is accessed
-  // as a raw buffer (slab_rsrc): the step and element select a scalar
-  // offset, the lane a fixed 32-bit offset.
-  // First half: nothing here waits on memory.
+  // Slabs.  Slab s is q after step s (slab 0: the initial condition).  With
+  // SEG = 1 the slabs 0 .. N/2 - 1 are all kept; with SEG > 1 every SEG-th, and
+  // the second half of the march recomputes the ones between from the kept
+  // one below them.  Kept slab number g starts at g * slab_len; within it row
+  // t of lane tid sits at (t / 2) * 2P + 2 tid + t % 2 (K >= 2: 16 bytes per
+  // lane and access) or at tid (K = 1).  Lanes whose rows are all padding
+  // (u0 >= n) store nothing (one exec mask for the whole loop) and load from
+  // lane 0's address, so a wave's dead lanes share one cache line; their
+  // values are replaced by 0.  The region is accessed as a raw buffer
+  // (slab_rsrc): the step and element select a scalar offset, the lane a fixed
+  // 32-bit offset.  First half: nothing here waits on memory.
   const bool lane_live = u0 < n;
   const __amdgpu_buffer_rsrc_t srsrc =
       slab_rsrc(slab, static_cast<unsigned>(a.slab_stride * sizeof(double)));
   const unsigned off_dst = static_cast<unsigned>(tid) * slab_lane_bytes<K>();
   const unsigned off_src = lane_live ? off_dst : 0u;
-  auto store_slab = [&](const int j) __attribute__((always_inline)) {
-    if (lane_live) slab_put<K>(q, srsrc, off_dst, static_cast<unsigned>(j * (P * K) * 8), P);
-  };
-  store_slab(0);
-  for (int j = 1; j < half; j++) {
-    advance();
-    store_slab(j);
-  }
-  // step N/2 pairs with itself
-  advance();
-  {
-    const double c0 = pw_lds[0];
+  constexpr unsigned SLAB_BYTES = march_slab_len(K, W, SEG) * 8u;
+  if constexpr (SEG == 1) {
+    auto store_slab = [&](const int j) __attribute__((always_inline)) {
+      if (lane_live) slab_put<K>(q, srsrc, off_dst, static_cast<unsigned>(j) * SLAB_BYTES, P);
+    };
+    for (int j = 0; j < half; j++) {
+      store_slab(j);
+      advance(q, ql, qr);
+    }
+    // step N/2 pairs with itself
+    {
+      const double c0 = pw[0];
 #pragma unroll
-    for (int t = 0; t < K; t++) acc[t] = c0 * q[t] * q[t];
-  }
+      for (int t = 0; t < K; t++) acc[t] = c0 * q[t] * q[t];
+    }
 
-  // Second half: step N/2 + i pairs with slab N/2 - i (i = 1 .. N/2).  Slabs
-  // come through a ring of PD register sets, each loaded PD steps before its
-  // use (indices below 0 reload slab 0 and are never used).  PD divides N/2
-  // (N is a power of two >= 16).
-  constexpr int PD = (K <= 2) ? 8 : (K == 4) ? 4 : 2;
-  double ring[PD][K];
-  auto fetch = [&](const int s, double (&dstv)[K]) __attribute__((always_inline)) {
-    slab_get<K>(dstv, srsrc, off_src, static_cast<unsigned>(max(s, 0) * (P * K) * 8), P);
-  };
-  // The loop below waits on each ring set by the count of loads issued after
-  // it.  That count is exact only if nothing else is in flight (the first
-  // half's slab stores are drained here) and the sets are issued in ring
-  // order (the scheduler may not reorder them across the barrier).
-  vmem_drain();
-#pragma unroll
-  for (int e = 0; e < PD; e++) {
-    fetch(half - 1 - e, ring[e]);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  for (int i0 = 1; i0 <= half; i0 += PD) {
+    // Second half: step N/2 + i pairs with slab N/2 - i (i = 1 .. N/2).  Slabs
+    // come through a ring of PD register sets, each loaded PD steps before its
+    // use (indices below 0 reload slab 0 and are never used).  PD divides N/2
+    // (N is a power of two >= 16).  What dead lanes load only ever multiplies
+    // their q = 0.
+    constexpr int PD = (K <= 2) ? 8 : (K == 4) ? 4 : 2;
+    double ring[PD][K];
+    auto fetch = [&](const int s, double (&dstv)[K]) __attribute__((always_inline)) {
+      slab_get<K>(dstv, srsrc, off_src, static_cast<unsigned>(max(s, 0)) * SLAB_BYTES, P);
+    };
+    // The loop below waits on each ring set by the count of loads issued after
+    // it.  That count is exact only if nothing else is in flight (the first
+    // half's slab stores are drained here) and the sets are issued in ring
+    // order (the scheduler may not reorder them across the barrier).
+    vmem_drain();
 #pragma unroll
     for (int e = 0; e < PD; e++) {
-      const int i = i0 + e;
-      advance();
-      const double cj = pw_lds[i];
+      fetch(half - 1 - e, ring[e]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // (a step's pairing stands before the next step, whose scans leave time
+    // for it; the step after N is computed and not used)
+    advance(q, ql, qr);
+    for (int i0 = 1; i0 <= half; i0 += PD) {
 #pragma unroll
-      for (int t = 0; t < K; t++) acc[t] = fma(cj * q[t], ring[e][t], acc[t]);
-      fetch(half - i - PD, ring[e]);
+      for (int e = 0; e < PD; e++) {
+        const int i = i0 + e;
+        const double cj = weight(i);
+#pragma unroll
+        for (int t = 0; t < K; t++) acc[t] = fma(cj * q[t], ring[e][t], acc[t]);
+        fetch(half - i - PD, ring[e]);
+        advance(q, ql, qr);
+      }
+    }
+  } else {
+    // A kept slab carries the values beyond each wave's two ends behind its
+    // rows (2 per wave): a step started from it needs them.
+    const unsigned off_edge =
+        static_cast<unsigned>(P * K + 2 * wave + (lane == 63 ? 1 : 0)) * 8u;
+    for (int g = 0; g < half / SEG; g++) {
+      const unsigned o = static_cast<unsigned>(g) * SLAB_BYTES;
+      if (lane_live) slab_put<K>(q, srsrc, off_dst, o, P);
+      if constexpr (W > 1) {
+        if (lane == 0 || lane == 63) slab_store(lane == 0 ? ql : qr, srsrc, off_edge, o);
+      }
+#pragma unroll 1
+      for (int e = 0; e < SEG; e++) advance(q, ql, qr);
+    }
+    {
+      const double c0 = pw[0];
+#pragma unroll
+      for (int t = 0; t < K; t++) acc[t] = c0 * q[t] * q[t];
+    }
+    // Second half, segment by segment: the slabs g SEG .. g SEG + SEG - 1 into
+    // this lane's own places in LDS (the kept one, loaded a segment ahead,
+    // then SEG - 1 steps from it: the same operations as in the first half, so
+    // the same bits), then SEG steps of the march that pair with them from the
+    // top down.
+    auto lds_slot = [&](const int e) __attribute__((always_inline)) {
+      return seg_lds + e * (P * K) + (K >= 2 ? 2 * tid : tid);
+    };
+    auto put_lds = [&](const double (&v)[K], const int e) __attribute__((always_inline)) {
+      double* d = lds_slot(e);
+      if constexpr (K >= 2) {
+#pragma unroll
+        for (int t = 0; t < K; t += 2)
+          *reinterpret_cast<f64x2*>(d + t * P) = f64x2{v[t], v[t + 1]};
+      } else {
+        d[0] = v[0];
+      }
+    };
+    double kept[K], edge = 0.0;
+    auto fetch = [&](const int g) __attribute__((always_inline)) {
+      const unsigned o = static_cast<unsigned>(max(g, 0)) * SLAB_BYTES;
+      slab_get<K>(kept, srsrc, off_src, o, P);
+      if constexpr (W > 1) edge = slab_load(srsrc, off_edge, o);
+    };
+    int g = half / SEG - 1;
+    fetch(g);
+    for (; g >= 0; g--) {
+      {
+        double s[K];
+#pragma unroll
+        for (int t = 0; t < K; t++) s[t] = lane_live ? kept[t] : 0.0;
+        double sl = wave_shr1(s[K - 1]), sr = wave_shl1(s[0]);
+        if constexpr (W > 1) {
+          sl = (lane == 0) ? edge : sl;
+          sr = (lane == 63) ? edge : sr;
+        }
+        put_lds(s, 0);
+        fetch(g - 1);
+#pragma unroll 1
+        for (int e = 1; e < SEG; e++) {
+          advance(s, sl, sr);
+          put_lds(s, e);
+        }
+      }
+#pragma unroll 1
+      for (int e = SEG - 1; e >= 0; e--) {
+        advance(q, ql, qr);
+        const double cj = weight(half - (g * SEG + e));
+        const double* p = lds_slot(e);
+        if constexpr (K >= 2) {
+#pragma unroll
+          for (int t = 0; t < K; t += 2) {
+            const f64x2 v = *reinterpret_cast<const f64x2*>(p + t * P);
+            acc[t] = fma(cj * q[t], v.x, acc[t]);
+            acc[t + 1] = fma(cj * q[t + 1], v.y, acc[t + 1]);
+          }
+        } else {
+          acc[0] = fma(cj * q[0], p[0], acc[0]);
+        }
+      }
     }
   }
 
@@ -530,11 +713,11 @@ __device__ void march_one(const MarchArgs& a, const int inst, const unsigned st0
 // instances converge.  Thread 0 takes the next index and broadcasts it
 // through LDS; the exit test is on that workgroup-uniform value, so every
 // wave leaves the loop together once the counter passes n_items.
-template <int K, int W>
-__global__ void __launch_bounds__(64 * W) march_kernel(MarchArgs a) {
+template <int K, int W, int SEG>
+__global__ void __launch_bounds__(64 * W, K == 8 ? 2 : 1) march_kernel(MarchArgs a) {
   __shared__ MarchShared<W> sh;
   __shared__ int s_next;
-  extern __shared__ double pw_lds[];  // half_max + 1 pairing weights
+  extern __shared__ __align__(16) double seg_lds[];  // SEG > 1: one segment's slabs
   const int tid = threadIdx.x;
   double* slab = a.slabs + (long long)blockIdx.x * a.slab_stride;
   for (;;) {
@@ -546,58 +729,112 @@ __global__ void __launch_bounds__(64 * W) march_kernel(MarchArgs a) {
     const int inst = __builtin_amdgcn_readfirstlane(a.items[it]);
     const unsigned st = __builtin_amdgcn_readfirstlane(a.status[inst]);
     if (st & ST_DONE_MASK) continue;
-    march_one<K, W>(a, inst, st, slab, sh, pw_lds, tid);
+    march_one<K, W, SEG>(a, inst, st, slab, sh, seg_lds, tid);
+  }
+}
+
+// The same queue for instances of up to 512 unknowns of any size, one wave
+// each: a sweep over many sizes then needs four launches for the four
+// hardware queues instead of seven, and no small bucket waits for another to
+// finish.  Costs the smallest sizes their occupancy (two waves per SIMD, the
+// registers of K = 8), so a batch that has queues left launches its buckets
+// one by one.
+template <int SEG>
+__global__ void __launch_bounds__(64, 2) march_small_kernel(MarchArgs a) {
+  __shared__ MarchShared<1> sh;
+  __shared__ int s_next;
+  extern __shared__ __align__(16) double seg_lds[];
+  const int tid = threadIdx.x;
+  double* slab = a.slabs + (long long)blockIdx.x * a.slab_stride;
+  for (;;) {
+    if (tid == 0) s_next = atomicAdd(a.queue, 1);
+    wg_barrier();
+    const int it = __builtin_amdgcn_readfirstlane(s_next);
+    wg_barrier();
+    if (it >= a.n_items) break;
+    const int inst = __builtin_amdgcn_readfirstlane(a.items[it]);
+    const unsigned st = __builtin_amdgcn_readfirstlane(a.status[inst]);
+    if (st & ST_DONE_MASK) continue;
+    const int n = __builtin_amdgcn_readfirstlane(a.desc[inst].n);
+    if (n <= 64)
+      march_one<1, 1, SEG>(a, inst, st, slab, sh, seg_lds, tid);
+    else if (n <= 128)
+      march_one<2, 1, SEG>(a, inst, st, slab, sh, seg_lds, tid);
+    else if (n <= 256)
+      march_one<4, 1, SEG>(a, inst, st, slab, sh, seg_lds, tid);
+    else
+      march_one<8, 1, SEG>(a, inst, st, slab, sh, seg_lds, tid);
   }
 }
 
 // ------------------------------------------------------------------ dispatch
-// (K, W) variants: K * 8 VGPRs of coefficients per lane must leave room for
-// the register file share of a 64W-lane workgroup (no spills).
+// (K, W) variants: one wave per instance up to 512 unknowns, then 4 or 8 rows
+// per lane.  Fewer rows per lane lose more to the scans than the shorter
+// lane-local passes give (a step of 512 unknowns: <8, 1> 0.29 us, <4, 2>
+// 0.35, <2, 4> 0.36), 16 spill.
 #define SCFT_MARCH_VARIANTS(X) \
-  X(1, 1) X(2, 1) X(4, 1) X(8, 1) X(16, 1) \
-  X(1, 2) X(2, 2) X(4, 2) X(8, 2) X(16, 2) \
-  X(1, 4) X(2, 4) X(4, 4) X(8, 4) X(16, 4) \
-  X(1, 8) X(2, 8) X(4, 8) X(8, 8)          \
-  X(1, 16) X(2, 16)
+  X(1, 1) X(2, 1) X(4, 1) X(8, 1) X(4, 2) X(8, 2) X(4, 4) X(8, 4) X(4, 8) X(8, 8)
 
-static size_t march_lds_bytes(int half_max) {
-  return static_cast<size_t>(half_max + 1) * sizeof(double);
-}
-
-static const void* march_fn(int K, int W) {
-#define X(k, w) \
-  if (K == k && W == w) return reinterpret_cast<const void*>(&march_kernel<k, w>);
+static const void* march_fn(int K, int W, int seg) {
+#define X(k, w)                                                                  \
+  if (K == k && W == w)                                                          \
+    return seg == 1 ? reinterpret_cast<const void*>(&march_kernel<k, w, 1>)      \
+                    : reinterpret_cast<const void*>(&march_kernel<k, w, MARCH_SEG>);
   SCFT_MARCH_VARIANTS(X)
 #undef X
   return nullptr;
 }
 
-bool march_variant_exists(int K, int W) { return march_fn(K, W) != nullptr; }
+static size_t march_lds_bytes(int K, int W, int seg) {
+  return seg > 1 ? static_cast<size_t>(seg) * 64 * W * K * sizeof(double) : 0;
+}
+
+bool march_variant_exists(int K, int W) { return march_fn(K, W, 1) != nullptr; }
 
 hipError_t launch_march(int K, int W, const MarchArgs& a, int grid, hipStream_t s) {
-#define X(k, w)                                                                 \
-  if (K == k && W == w) {                                                       \
-    hipLaunchKernelGGL((march_kernel<k, w>), dim3(grid), dim3(64 * w),           \
-                       march_lds_bytes(a.half_max), s, a);                      \
-    return hipGetLastError();                                                   \
+  const size_t lds = march_lds_bytes(K, W, a.seg);
+#define X(k, w)                                                                          \
+  if (K == k && W == w) {                                                                \
+    if (a.seg == 1)                                                                      \
+      hipLaunchKernelGGL((march_kernel<k, w, 1>), dim3(grid), dim3(64 * w), lds, s, a);  \
+    else                                                                                 \
+      hipLaunchKernelGGL((march_kernel<k, w, MARCH_SEG>), dim3(grid), dim3(64 * w), lds, \
+                         s, a);                                                          \
+    return hipGetLastError();                                                            \
   }
   SCFT_MARCH_VARIANTS(X)
 #undef X
   return hipErrorInvalidValue;
 }
 
-int march_max_grid(int K, int W, int half_max) {
-  const void* f = march_fn(K, W);
-  if (!f) return 0;
+static int resident_grid(const void* f, int threads, size_t lds) {
   int dev = 0, cus = 0, per = 0;
   if (hipGetDevice(&dev) != hipSuccess) return 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     return 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, f, 64 * W, march_lds_bytes(half_max)) !=
-      hipSuccess)
-    return 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, f, threads, lds) != hipSuccess) return 0;
   if (per < 1) per = 1;
   return per * cus;
+}
+
+int march_max_grid(int K, int W, int seg) {
+  const void* f = march_fn(K, W, seg);
+  return f ? resident_grid(f, 64 * W, march_lds_bytes(K, W, seg)) : 0;
+}
+
+hipError_t launch_march_small(const MarchArgs& a, int grid, hipStream_t s) {
+  const size_t lds = march_lds_bytes(8, 1, a.seg);
+  if (a.seg == 1)
+    hipLaunchKernelGGL(march_small_kernel<1>, dim3(grid), dim3(64), lds, s, a);
+  else
+    hipLaunchKernelGGL(march_small_kernel<MARCH_SEG>, dim3(grid), dim3(64), lds, s, a);
+  return hipGetLastError();
+}
+
+int march_small_max_grid(int seg) {
+  const void* f = seg == 1 ? reinterpret_cast<const void*>(&march_small_kernel<1>)
+                           : reinterpret_cast<const void*>(&march_small_kernel<MARCH_SEG>);
+  return resident_grid(f, 64, march_lds_bytes(8, 1, seg));
 }
 
 }  // namespace scft

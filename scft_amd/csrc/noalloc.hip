@@ -92,7 +92,7 @@ extern "C" int scft_eval_noalloc(int M, int N, int bc, int cmat, const double* d
   if (N < 16 || N > 16384 || (N & (N - 1)) != 0)
     return fail(SCFT_E_ARG, "N must be a power of two in [16, 16384]");
   const int cap = bucket_capacity(n);
-  const int K = bucket_default_K(cap, false), W = cap / 64 / K;
+  const int K = bucket_default_K(cap, false, 1, 1), W = cap / 64 / K;
   const long long slab_doubles = static_cast<long long>(N / 2) * cap;
   if (static_cast<size_t>(slab_doubles) * sizeof(double) > kSlabBytes) {
     snprintf(g_msg, sizeof g_msg,
@@ -145,6 +145,7 @@ extern "C" int scft_eval_noalloc(int M, int N, int bc, int cmat, const double* d
   a.queue = reinterpret_cast<int*>(base + kQueueOff);
   a.n_items = 1;
   a.half_max = N / 2;
+  a.seg = 1;
   e = launch_march(K, W, a, 1, s);
   if (e != hipSuccess) return fail(SCFT_E_HIP, "march launch", e);
   // the host staging buffer is reused by the next call: wait for this one

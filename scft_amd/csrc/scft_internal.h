@@ -38,7 +38,8 @@ struct MarchArgs {
   const int* items;       // instance ids of this bucket, largest first
   int* queue;             // next item to take (zeroed before every launch)
   int n_items;
-  int half_max;           // largest N/2 of the bucket (LDS weight table size - 1)
+  int half_max;           // largest N/2 of the bucket (IRK4: LDS weight table size - 1)
+  int seg;                // 1: every slab is kept, MARCH_SEG: every MARCH_SEG-th (march.hip)
 };
 
 constexpr unsigned ST_CONVERGED = 1u;
@@ -106,19 +107,32 @@ inline int bucket_capacity(int n) {
   while (c < n) c *= 2;
   return c;
 }
-// Rows per lane of a bucket before any tuning: implicit Euler keeps ~8
-// doubles per row in registers, IRK4 ~11 (its variants stop at K = 8).
-inline int bucket_default_K(int cap, bool irk4) {
-  const int k = cap / 64, kmax = irk4 ? 8 : 16;
-  return k < kmax ? k : kmax;
+// Rows per lane of a bucket of `items` instances before any tuning.  Implicit
+// Euler: one wave up to 512 unknowns, then waves of 8 rows per lane; the 1024
+// bucket takes 4 waves of 4 rows while every instance finds a CU of its own
+// (a step 0.37 us against 0.47 us at <8, 2>), and <8, 2> beyond (1030 against
+// 860 G node-steps/s with the chip full).  IRK4 keeps ~11 doubles per row.
+inline int bucket_default_K(int cap, bool irk4, int items, int cus) {
+  if (!irk4 && cap == 1024 && items <= cus) return 4;
+  const int k = cap / 64;
+  return k < 8 ? k : 8;
 }
+
+// Slabs of a workgroup that keeps every seg-th, and the doubles of one kept
+// slab (seg > 1: two more per wave).
+constexpr int MARCH_SEG = 4;
+constexpr int march_slab_len(int K, int W, int seg) { return 64 * W * K + (seg > 1 ? 2 * W : 0); }
 
 // Launch one bucket.  Returns hipSuccess or the launch error.
 hipError_t launch_march(int K, int W, const MarchArgs& a, int grid,
                         hipStream_t s);
 // Largest grid of co-resident workgroups for a variant (persistent launch).
-int march_max_grid(int K, int W, int half_max);
+int march_max_grid(int K, int W, int seg);
 bool march_variant_exists(int K, int W);
+// Instances of up to 512 unknowns of any size in one launch of single waves
+// (rows per lane by n, as bucket_default_K).
+hipError_t launch_march_small(const MarchArgs& a, int grid, hipStream_t s);
+int march_small_max_grid(int seg);
 // The same for the two-stage Gauss (IRK4) march (irk4.hip).
 hipError_t launch_irk4(int K, int W, const MarchArgs& a, int grid, hipStream_t s);
 int irk4_max_grid(int K, int W, int half_max);  // 0: the workgroup does not fit
