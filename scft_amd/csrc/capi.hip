@@ -64,6 +64,7 @@ struct Bucket {
   std::vector<int> items;  // instance ids, largest cost first
   int* d_items = nullptr;
   int grid = 0;
+  int dense = 0;  // width of the dense march (dense.hip), 0: the scan march
   int wpc = 0;  // workgroups per CU of the persistent grid (0: as many as fit)
   long long slab_stride = 0;  // doubles per workgroup
   long long slab_base = 0;    // this bucket's region in the scratch (doubles)
@@ -182,6 +183,9 @@ static double step_us(int K, int W) {
 // A persistent grid's expected run: its longest instance, or all of them
 // spread over the workgroups.
 static double run_us(const scft_batch* b, const Bucket& bk, int grid) {
+  if (bk.dense)  // ~35 / 110 us to build the powers, then 64 steps at a time
+    return (bk.dense == 32 ? 35.0 + 0.008 * bk.Nmax : 110.0 + 0.03 * bk.Nmax) *
+           ((bk.items.size() + grid - 1) / std::max(1, grid));
   double steps = 0.0;
   for (int k : bk.items) steps += b->desc[k].N;
   return step_us(bk.K, bk.W) * std::max<double>(bk.Nmax, steps / std::max(1, grid));
@@ -193,6 +197,8 @@ static int size_scratch(scft_batch* b) {
   drop_sweep_graph(b);
   const bool irk4 = b->stepper == SCFT_STEP_IRK4;
   auto grid_of = [&](const Bucket& bk, int seg) {
+    if (bk.dense)
+      return std::min<int>(static_cast<int>(bk.items.size()), dense_max_grid(bk.dense, irk4));
     const int mg = eval_max_grid(b, bk.K, bk.W, bk.Nmax / 2, seg);
     // fewer co-resident workgroups per CU can finish a bucket sooner: its
     // longest instances set the makespan, and they step faster alone
@@ -200,6 +206,7 @@ static int size_scratch(scft_batch* b) {
     return std::min<int>(static_cast<int>(bk.items.size()), cap_grid);
   };
   int filled = 0, small = 0;
+  for (auto& bk : b->buckets) filled += bk.items.empty() ? 0 : 1;
   bool small_ok = !irk4;
   double longest = 0.0;
   for (auto& bk : b->buckets) {
@@ -208,13 +215,18 @@ static int size_scratch(scft_batch* b) {
       snprintf(g_errmsg, sizeof g_errmsg, "no march variant K=%d W=%d", bk.K, bk.W);
       return SCFT_E_ARG;
     }
+    bk.dense = 0;
+    if (bk.cap == 64 && filled <= 1 + scft_batch::kSide) {
+      int Nmin = bk.Nmax;
+      for (int k : bk.items) Nmin = std::min(Nmin, b->desc[k].N);
+      bk.dense = dense_width(bk.nmax, Nmin, static_cast<int>(bk.items.size()), b->cus, irk4);
+    }
     const int g = grid_of(bk, 1);
     if (g < 1) {
       snprintf(g_errmsg, sizeof g_errmsg, "march variant K=%d W=%d does not fit a CU", bk.K,
                bk.W);
       return SCFT_E_ARG;
     }
-    filled++;
     if (bk.cap <= 512) {
       small++;
       small_ok = small_ok && bk.W == 1 && bk.K == bk.cap / 64 && bk.wpc == 0;
@@ -245,7 +257,8 @@ static int size_scratch(scft_batch* b) {
     const bool in_group = merge && bk.cap <= 512;
     bk.grid = std::max(1, grid_of(bk, b->seg));
     const long long kept = std::max(1, bk.Nmax / 2 / b->seg);
-    bk.slab_stride = kept * march_slab_len(bk.K, bk.W, b->seg);
+    bk.slab_stride = bk.dense ? static_cast<long long>(bk.Nmax / 2) * bk.dense
+                              : kept * march_slab_len(bk.K, bk.W, b->seg);
     bk.slab_base = need;
     double work = 0.0;
     for (int k : bk.items) work += static_cast<double>(b->desc[k].n) * b->desc[k].N;
@@ -369,6 +382,12 @@ static MarchArgs march_args(const scft_batch* b, const Bucket& bk, int bucket_id
   return a;
 }
 
+static hipError_t launch_bucket(scft_batch* b, const Bucket& bk, const MarchArgs& a, int grid,
+                                hipStream_t s) {
+  return bk.dense ? launch_dense(bk.dense, b->stepper == SCFT_STEP_IRK4, a, grid, s)
+                  : launch_eval(b, bk.K, bk.W, a, grid, s);
+}
+
 static hipError_t launch_part(scft_batch* b, const Launch& l, hipStream_t s) {
   const Bucket& bk = b->buckets[l.bucket];
   MarchArgs a = march_args(b, bk, l.bucket);
@@ -377,7 +396,7 @@ static hipError_t launch_part(scft_batch* b, const Launch& l, hipStream_t s) {
   a.half_max = l.Nmax / 2;
   a.items = l.d_items;
   a.n_items = l.n_items;
-  return l.small ? launch_march_small(a, l.grid, s) : launch_eval(b, bk.K, bk.W, a, l.grid, s);
+  return l.small ? launch_march_small(a, l.grid, s) : launch_bucket(b, bk, a, l.grid, s);
 }
 
 // One evaluation sweep of every instance not marked done: counters reset on
@@ -727,12 +746,12 @@ extern "C" int scft_batch_time_buckets(scft_batch* b, const double* w, int reps,
     if (bk.items.empty()) continue;
     const MarchArgs a = march_args(b, bk, i);
     HIPCHK(launch_reset(b->d_counters, nb + 1, b->stream));
-    HIPCHK(launch_eval(b, bk.K, bk.W, a, bk.grid, b->stream));  // warm-up
+    HIPCHK(launch_bucket(b, bk, a, bk.grid, b->stream));  // warm-up
     HIPCHK(hipEventRecord(e0, b->stream));
     for (int r = 0; r < reps; r++) {
       // the counter reset is a ~2 us kernel inside the timed region
       HIPCHK(launch_reset(b->d_counters, nb + 1, b->stream));
-      HIPCHK(launch_eval(b, bk.K, bk.W, a, bk.grid, b->stream));
+      HIPCHK(launch_bucket(b, bk, a, bk.grid, b->stream));
     }
     HIPCHK(hipEventRecord(e1, b->stream));
     HIPCHK(hipEventSynchronize(e1));
@@ -836,7 +855,7 @@ extern "C" int scft_batch_autotune(scft_batch* b, int reps) {
   const int nb = static_cast<int>(b->buckets.size());
   for (int bi = 0; bi < nb; bi++) {
     Bucket& bk = b->buckets[bi];
-    if (bk.items.empty()) continue;
+    if (bk.items.empty() || bk.dense) continue;  // (the dense march has one variant)
     float best = 1e30f;
     int bestK = bk.K, bestW = bk.W, bestP = bk.wpc;
     for (int K : Ks)
@@ -908,6 +927,17 @@ extern "C" int scft_debug_slabs(scft_batch* b, int inst, double* out) {
   for (auto& bk : b->buckets) {
     if (bk.items.empty()) continue;
     const int P = 64 * bk.W, K = bk.K, half = d.N / 2;  // one instance: every slab is kept
+    if (bk.dense) {  // blocks of 64 steps: rows by four, 16 steps side by side (dense.hip)
+      std::vector<double> raw(static_cast<size_t>(half) * bk.dense);
+      HIPCHK(hipMemcpy(raw.data(), b->d_slabs + bk.slab_base, raw.size() * sizeof(double),
+                       hipMemcpyDeviceToHost));
+      for (int s = 1; s < half; s++)
+        for (int u = 0; u < d.n; u++)
+          out[static_cast<size_t>(s - 1) * d.n + u] =
+              raw[(static_cast<size_t>(s / 16) * (bk.dense / 4) + u / 4) * 64 + u % 4 * 16 +
+                  s % 16];
+      return SCFT_OK;
+    }
     std::vector<double> raw(static_cast<size_t>(half) * P * K);
     HIPCHK(hipMemcpy(raw.data(), b->d_slabs + bk.slab_base, raw.size() * sizeof(double),
                      hipMemcpyDeviceToHost));

@@ -135,6 +135,28 @@ __device__ __forceinline__ void slab_get(double (&d)[K], __amdgpu_buffer_rsrc_t 
   }
 }
 
+// ---- complex FP64
+struct cd {
+  double re, im;
+};
+__device__ __forceinline__ cd c_add(cd a, cd b) { return {a.re + b.re, a.im + b.im}; }
+__device__ __forceinline__ cd c_mul(cd a, cd b) {
+  return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
+}
+// a * b + c
+__device__ __forceinline__ cd c_fma(cd a, cd b, cd c) {
+  return {fma(a.re, b.re, fma(-a.im, b.im, c.re)), fma(a.re, b.im, fma(a.im, b.re, c.im))};
+}
+// c - a * b
+__device__ __forceinline__ cd c_fnma(cd a, cd b, cd c) {
+  return {fma(-a.re, b.re, fma(a.im, b.im, c.re)), fma(-a.re, b.im, fma(-a.im, b.re, c.im))};
+}
+__device__ __forceinline__ cd c_div(cd a, cd b) {
+  const double s = 1.0 / (b.re * b.re + b.im * b.im);
+  return {(a.re * b.re + a.im * b.im) * s, (a.im * b.re - a.re * b.im) * s};
+}
+__device__ __forceinline__ cd c_sel(bool p, cd a, cd b) { return {p ? a.re : b.re, p ? a.im : b.im}; }
+
 // ---- double-double arithmetic (hi + lo, |lo| <= ulp(hi)/2) for the pivot
 // scan.  The pivots are a projective product of 2x2 matrices whose two
 // eigenvalues nearly coincide when diffusion dominates (dt/h^2 >> 1); in FP64

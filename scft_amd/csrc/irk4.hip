@@ -35,30 +35,11 @@
 // the lane moves; the HBM traffic per evaluation is the same.
 #include "scft_internal.h"
 #include "device_common.h"
+#include "march_rows.h"
 
 namespace scft {
 
-// ------------------------------------------------------------ complex FP64
-struct cd {
-  double re, im;
-};
-__device__ __forceinline__ cd c_add(cd a, cd b) { return {a.re + b.re, a.im + b.im}; }
-__device__ __forceinline__ cd c_mul(cd a, cd b) {
-  return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
-}
-// a * b + c
-__device__ __forceinline__ cd c_fma(cd a, cd b, cd c) {
-  return {fma(a.re, b.re, fma(-a.im, b.im, c.re)), fma(a.re, b.im, fma(a.im, b.re, c.im))};
-}
-// c - a * b
-__device__ __forceinline__ cd c_fnma(cd a, cd b, cd c) {
-  return {fma(-a.re, b.re, fma(a.im, b.im, c.re)), fma(-a.re, b.im, fma(-a.im, b.re, c.im))};
-}
-__device__ __forceinline__ cd c_div(cd a, cd b) {
-  const double s = 1.0 / (b.re * b.re + b.im * b.im);
-  return {(a.re * b.re + a.im * b.im) * s, (a.im * b.re - a.re * b.im) * s};
-}
-__device__ __forceinline__ cd c_sel(bool p, cd a, cd b) { return {p ? a.re : b.re, p ? a.im : b.im}; }
+// ------------------------------------------------------------ lane moves of complex values
 template <int S>
 __device__ __forceinline__ cd c_row_shr(cd v) { return {row_shr<S>(v.re), row_shr<S>(v.im)}; }
 template <int S>
@@ -130,53 +111,6 @@ struct Irk4Shared {
   double red[W];     // norm reduction
   unsigned bad[W];
 };
-
-// Rows of the mass matrix A and of D' = B + C for unknown u (node u+1), from
-// its two adjacent elements; the same expressions and boundary handling as
-// march.hip's assemble_row (no FMA contraction).  Padding rows (u >= n) are
-// zero in both, and the couplings to Dirichlet nodes or past the last
-// unknown are dropped.
-struct SplitRow {
-  double al, ad, ar;  // A
-  double dl, dd, dr;  // D'
-};
-__device__ __forceinline__ SplitRow assemble_split(const double* __restrict__ x,
-                                                   const double* __restrict__ w, int n, int M,
-                                                   int u, int cmat, double wall0, double wallL) {
-#pragma clang fp contract(off)
-  const bool live = u < n;
-  const int i = live ? u + 1 : 1;
-  const double xl = x[i - 1], xc = x[i];
-  const bool has_r = (i + 1 < M);
-  const double xr = has_r ? x[i + 1] : xc;
-  const double hl = xc - xl, hr = xr - xc;
-  const double wi = live ? w[live ? u : 0] : 0.0;
-  const double Al = hl / 6.0, Ar = hr / 6.0, Ad = hl / 3.0 + hr / 3.0;
-  const double Bl = -1.0 / hl;
-  const double Br = has_r ? -1.0 / hr : 0.0;
-  const double Bd = 1.0 / hl + (has_r ? 1.0 / hr : 0.0);
-  double Cl, Cd, Cr;
-  if (cmat == 0) {
-    Cl = wi * Al;
-    Cd = wi * Ad;
-    Cr = wi * Ar;
-  } else {
-    const double wl = (u > 0 && live) ? w[u - 1] : wall0;
-    const double wr = (u + 1 < n) ? w[u + 1] : wallL;
-    Cl = hl * (wl + wi) / 12.0;
-    Cd = hl * (wl + 3.0 * wi) / 12.0 + hr * (3.0 * wi + wr) / 12.0;
-    Cr = hr * (wi + wr) / 12.0;
-  }
-  const bool has_l = live && u > 0, has_rr = live && u < n - 1;
-  SplitRow s;
-  s.al = has_l ? Al : 0.0;
-  s.ad = live ? Ad : 0.0;
-  s.ar = has_rr ? Ar : 0.0;
-  s.dl = has_l ? Bl + Cl : 0.0;
-  s.dd = live ? Bd + Cd : 0.0;
-  s.dr = has_rr ? Br + Cr : 0.0;
-  return s;
-}
 
 template <int K, int W>
 __device__ void irk4_one(const MarchArgs& a, const int inst, const unsigned st0,

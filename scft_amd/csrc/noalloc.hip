@@ -146,7 +146,8 @@ extern "C" int scft_eval_noalloc(int M, int N, int bc, int cmat, const double* d
   a.n_items = 1;
   a.half_max = N / 2;
   a.seg = 1;
-  e = launch_march(K, W, a, 1, s);
+  const int np = dense_width(n, N, 1, 1, false);
+  e = np ? launch_dense(np, false, a, 1, s) : launch_march(K, W, a, 1, s);
   if (e != hipSuccess) return fail(SCFT_E_HIP, "march launch", e);
   // the host staging buffer is reused by the next call: wait for this one
   e = hipStreamSynchronize(s);

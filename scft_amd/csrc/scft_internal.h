@@ -133,6 +133,28 @@ bool march_variant_exists(int K, int W);
 // (rows per lane by n, as bucket_default_K).
 hipError_t launch_march_small(const MarchArgs& a, int grid, hipStream_t s);
 int march_small_max_grid(int seg);
+// Instances of up to 64 unknowns as dense products on the matrix cores, 32 or
+// 64 unknowns wide (dense.hip); kept slabs: N/2 x width doubles.
+hipError_t launch_dense(int np, bool irk4, const MarchArgs& a, int grid, hipStream_t s);
+int dense_max_grid(int np, bool irk4);
+constexpr int DENSE_COLS = 64;  // steps per block
+// Width for `items` instances of at most n unknowns and at least N steps, or 0:
+// the scan march.  The powers cost 30-40 us (width 32) or 100-120 us, then 64
+// steps take 0.5 or 1.8 us, one workgroup of each CU at a time; a scan step
+// takes 0.15 us (IRK4 0.31) however many there are, up to 1024 waves.  Sweeps
+// of 1 / 512 / 1024 / 4096 instances in us, dense against scan:
+//   n = 31, N = 256   37 /  59 / 102 / 357       52 /  65 /  81 / 182
+//           N = 512   39 /  65 / 112 / 399       89 / 115 / 129 / 301
+//           N = 1024  43 /  76 / 128 / 461      163 / 212 / 223 / 534
+//   n = 59, N = 1024 145 / 307 /   - /   -      163 / 180 / 201 / 639
+//   n = 59, N = 512, IRK4, 158 / 332 against 180 / 202.
+inline int dense_width(int n, int N, int items, int cus, bool irk4) {
+  if (n <= 32) {
+    const int most = N >= 1024 || (irk4 && N >= 512) ? items : N >= 512 ? 4 * cus : 2 * cus;
+    return N >= 256 && items <= most ? 32 : 0;
+  }
+  return n <= 64 && N >= (irk4 ? 512 : 1024) && items <= cus ? 64 : 0;
+}
 // The same for the two-stage Gauss (IRK4) march (irk4.hip).
 hipError_t launch_irk4(int K, int W, const MarchArgs& a, int grid, hipStream_t s);
 int irk4_max_grid(int K, int W, int half_max);  // 0: the workgroup does not fit
