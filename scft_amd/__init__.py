@@ -270,6 +270,9 @@ class Batch:
         tot = C.c_longlong()
         check(lib.scft_batch_layout(self.h, self.uoff, C.byref(tot)), "scft_batch_layout")
         self.total = tot.value
+        # (an evaluation's outputs are cut twice: plain integers, once)
+        self._rows = int(self.n[0]) if (self.n == self.n[0]).all() else 0
+        self._cuts = [slice(o, o + n) for o, n in zip(self.uoff.tolist(), self.n.tolist())]
 
     def close(self):
         if getattr(self, "h", None):
@@ -283,7 +286,10 @@ class Batch:
             pass
 
     def split(self, flat):
-        return [flat[o:o + n] for o, n in zip(self.uoff, self.n)]
+        if self._rows and isinstance(flat, np.ndarray) and flat.shape == (self.total,):
+            # instances of one size: the rows of a matrix
+            return list(flat.reshape(len(self.n), self._rows))
+        return [flat[s] for s in self._cuts]
 
     def join(self, parts):
         """Concatenated unknowns of all instances (a flat array passes through).

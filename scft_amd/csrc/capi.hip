@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <cstdint>
 #include <cstdio>
 #include <cstring>
 #include <fstream>
@@ -86,6 +87,8 @@ struct Launch {
 
 }  // namespace
 
+constexpr size_t kStageBytes = size_t(256) << 10;
+
 struct scft_batch {
   int device = 0;
   int n_inst = 0;
@@ -106,13 +109,20 @@ struct scft_batch {
   // queue runs its kernels one after the other, whichever the runtime put
   // there.  With four streams the pairing is ours (size_scratch).
   static constexpr int kSide = 3;
+  bool queued = false;  // some launch has more items than workgroups: its queue is reset
   hipStream_t side[kSide] = {};
   hipEvent_t fork = nullptr, join[kSide] = {};
   // device state
   InstDesc* d_desc = nullptr;
-  double *d_x = nullptr, *d_w = nullptr, *d_phit = nullptr, *d_pw = nullptr;
-  double *d_phi = nullptr, *d_r = nullptr, *d_rnorm = nullptr;
+  double *d_x = nullptr, *d_phit = nullptr, *d_pw = nullptr;
+  // field, status, ||r||, residual and density, one after the other in d_io:
+  // an evaluation's inputs and outputs are one copy each
+  unsigned char* d_io = nullptr;
+  double *d_w = nullptr, *d_phi = nullptr, *d_r = nullptr, *d_rnorm = nullptr;
   unsigned* d_status = nullptr;
+  size_t off_status = 0, off_rnorm = 0, off_r = 0, off_phi = 0, io_bytes = 0;
+  unsigned char* h_io = nullptr;  // pinned: all of it up to kStageBytes, else to ||r||
+  bool staged = false;
   double* d_slabs = nullptr;
   long long slab_doubles = 0;
   int* d_counters = nullptr;  // bucket queues, the active count, then a slot the
@@ -319,8 +329,10 @@ static int size_scratch(scft_batch* b) {
                    [](const Launch& p, const Launch& q) { return p.us > q.us; });
   double load[1 + scft_batch::kSide] = {};
   b->top_launch = -1;
+  b->queued = false;
   for (size_t i = 0; i < b->launches.size(); i++) {
     Launch& l = b->launches[i];
+    b->queued = b->queued || l.n_items > l.grid;
     for (int t = 1; t <= scft_batch::kSide; t++)
       if (load[t] < load[l.stream]) l.stream = t;
     load[l.stream] += l.us;
@@ -411,7 +423,11 @@ static hipStream_t stream_of(scft_batch* b, int s) { return s == 0 ? b->stream :
 
 static int enqueue_sweep(scft_batch* b) {
   const int nb = static_cast<int>(b->buckets.size());
-  HIPCHK(launch_reset(b->d_counters, nb + 1, b->stream));
+  if (b->queued) HIPCHK(launch_reset(b->d_counters, nb + 1, b->stream));
+  if (b->launches.size() == 1) {
+    HIPCHK(launch_part(b, b->launches[0], b->stream));
+    return SCFT_OK;
+  }
   bool used[1 + scft_batch::kSide] = {true};
   for (auto& l : b->launches) used[l.stream] = true;
   HIPCHK(hipEventRecord(b->fork, b->stream));
@@ -590,13 +606,28 @@ extern "C" int scft_batch_create(scft_batch** out, const scft_batch_desc* dsc) {
       return fail(SCFT_E_HIP);
   if (hipEventCreateWithFlags(&b->fork, hipEventDisableTiming) != hipSuccess)
     return fail(SCFT_E_HIP);
+  {
+    const size_t field = sizeof(double) * b->total_u;
+    b->off_status = field;
+    b->off_rnorm = b->off_status + (sizeof(unsigned) * b->n_inst + 7) / 8 * 8;
+    b->off_r = b->off_rnorm + sizeof(double) * b->n_inst;
+    b->off_phi = b->off_r + field;
+    b->io_bytes = b->off_phi + field;
+    b->staged = b->io_bytes <= kStageBytes;
+  }
   if ((rc = dalloc(&b->d_desc, b->n_inst)) || (rc = dalloc(&b->d_x, b->total_x)) ||
-      (rc = dalloc(&b->d_w, b->total_u)) || (rc = dalloc(&b->d_phit, b->total_u)) ||
-      (rc = dalloc(&b->d_pw, b->total_pw)) || (rc = dalloc(&b->d_phi, b->total_u)) ||
-      (rc = dalloc(&b->d_r, b->total_u)) || (rc = dalloc(&b->d_rnorm, b->n_inst)) ||
-      (rc = dalloc(&b->d_status, b->n_inst)) ||
+      (rc = dalloc(&b->d_io, b->io_bytes)) || (rc = dalloc(&b->d_phit, b->total_u)) ||
+      (rc = dalloc(&b->d_pw, b->total_pw)) ||
       (rc = dalloc(&b->d_counters, b->buckets.size() + 2)))
     return fail(rc);
+  b->d_w = reinterpret_cast<double*>(b->d_io);
+  b->d_status = reinterpret_cast<unsigned*>(b->d_io + b->off_status);
+  b->d_rnorm = reinterpret_cast<double*>(b->d_io + b->off_rnorm);
+  b->d_r = reinterpret_cast<double*>(b->d_io + b->off_r);
+  b->d_phi = reinterpret_cast<double*>(b->d_io + b->off_phi);
+  if (hipHostMalloc(reinterpret_cast<void**>(&b->h_io),
+                    b->staged ? b->io_bytes : b->off_r - b->off_status) != hipSuccess)
+    return fail(SCFT_E_NOMEM);
   for (auto& bk : b->buckets) {
     if (bk.items.empty()) continue;
     if ((rc = dalloc(&bk.d_items, bk.items.size()))) return fail(rc);
@@ -629,13 +660,10 @@ extern "C" int scft_batch_destroy(scft_batch* b) {
   for (auto& bk : b->buckets) dfree(bk.d_items);
   dfree(b->d_desc);
   dfree(b->d_x);
-  dfree(b->d_w);
   dfree(b->d_phit);
   dfree(b->d_pw);
-  dfree(b->d_phi);
-  dfree(b->d_r);
-  dfree(b->d_rnorm);
-  dfree(b->d_status);
+  dfree(b->d_io);
+  if (b->h_io) (void)hipHostFree(b->h_io);
   dfree(b->d_slabs);
   dfree(b->d_counters);
   dfree(b->d_hw);
@@ -686,25 +714,52 @@ static int batch_set_target(scft_batch* b, const double* phit) {
   return SCFT_OK;
 }
 
+// Touch the pages of an output array that a copy is about to fill (their
+// contents stay): a fresh array's page faults, 0.3 us each, then pass while the
+// device computes.
+static void touch_pages(void* p, size_t bytes) {
+  if (bytes < (size_t(1) << 20)) return;
+  volatile char* c = static_cast<volatile char*>(p);
+  volatile char* const end = c + bytes;
+  for (; c < end; c = reinterpret_cast<volatile char*>(
+                      (reinterpret_cast<uintptr_t>(c) | 4095) + 1))
+    *c = *c;
+}
+
 static int batch_eval_impl(scft_batch* b, const double* w, double* phi, double* r,
                            double* rnorm, unsigned* status) {
-  HIPCHK(hipMemcpyAsync(b->d_w, w, sizeof(double) * b->total_u, hipMemcpyHostToDevice,
-                        b->stream));
+  const size_t field = sizeof(double) * b->total_u;
+  // statuses start at zero
+  if (b->staged) {
+    // Small batches: one copy in, one out, through pinned memory (five copies
+    // of pageable memory took 60-80 us of a 130 us call).
+    std::memcpy(b->h_io, w, field);
+    std::memset(b->h_io + b->off_status, 0, b->off_rnorm - b->off_status);
+    HIPCHK(hipMemcpyAsync(b->d_io, b->h_io, b->off_rnorm, hipMemcpyHostToDevice, b->stream));
+    SCFT_TRY(enqueue_sweep(b));
+    const size_t end = phi ? b->io_bytes : b->off_phi;
+    HIPCHK(hipMemcpyAsync(b->h_io + b->off_status, b->d_io + b->off_status, end - b->off_status,
+                          hipMemcpyDeviceToHost, b->stream));
+    HIPCHK(hipStreamSynchronize(b->stream));
+    if (phi) std::memcpy(phi, b->h_io + b->off_phi, field);
+    if (r) std::memcpy(r, b->h_io + b->off_r, field);
+    if (rnorm) std::memcpy(rnorm, b->h_io + b->off_rnorm, sizeof(double) * b->n_inst);
+    if (status) std::memcpy(status, b->h_io + b->off_status, sizeof(unsigned) * b->n_inst);
+    return SCFT_OK;
+  }
+  HIPCHK(hipMemcpyAsync(b->d_w, w, field, hipMemcpyHostToDevice, b->stream));
   HIPCHK(hipMemsetAsync(b->d_status, 0, sizeof(unsigned) * b->n_inst, b->stream));
   SCFT_TRY(enqueue_sweep(b));
-  if (phi)
-    HIPCHK(hipMemcpyAsync(phi, b->d_phi, sizeof(double) * b->total_u, hipMemcpyDeviceToHost,
-                          b->stream));
-  if (r)
-    HIPCHK(hipMemcpyAsync(r, b->d_r, sizeof(double) * b->total_u, hipMemcpyDeviceToHost,
-                          b->stream));
-  if (rnorm)
-    HIPCHK(hipMemcpyAsync(rnorm, b->d_rnorm, sizeof(double) * b->n_inst, hipMemcpyDeviceToHost,
-                          b->stream));
-  if (status)
-    HIPCHK(hipMemcpyAsync(status, b->d_status, sizeof(unsigned) * b->n_inst,
-                          hipMemcpyDeviceToHost, b->stream));
+  HIPCHK(hipMemcpyAsync(b->h_io, b->d_io + b->off_status, b->off_r - b->off_status,
+                        hipMemcpyDeviceToHost, b->stream));
+  if (phi) touch_pages(phi, field);
+  if (r) touch_pages(r, field);
+  if (phi) HIPCHK(hipMemcpyAsync(phi, b->d_phi, field, hipMemcpyDeviceToHost, b->stream));
+  if (r) HIPCHK(hipMemcpyAsync(r, b->d_r, field, hipMemcpyDeviceToHost, b->stream));
   HIPCHK(hipStreamSynchronize(b->stream));
+  if (rnorm)
+    std::memcpy(rnorm, b->h_io + (b->off_rnorm - b->off_status), sizeof(double) * b->n_inst);
+  if (status) std::memcpy(status, b->h_io, sizeof(unsigned) * b->n_inst);
   return SCFT_OK;
 }
 
@@ -1102,6 +1157,7 @@ extern "C" int scft_batch_solve_resident(scft_batch* b, const scft_anderson_opts
   HIPCHK(hipMemsetAsync(b->d_iters, 0, sizeof(int) * b->n_inst, b->stream));
 
   // first sweep eagerly: the warm-start fallback needs the median first residual
+  HIPCHK(launch_reset(b->d_counters, nb + 1, b->stream));  // (the active count too)
   SCFT_TRY(enqueue_sweep(b));
   if (b->has_wcold && o->fallback_factor > 0.0) {
     std::vector<double> rn(b->n_inst);
@@ -1175,9 +1231,11 @@ extern "C" int scft_batch_solve_resident(scft_batch* b, const scft_anderson_opts
 extern "C" int scft_batch_download(scft_batch* b, double* w, int* iters, unsigned* status,
                                    scft_solve_stats* stats) {
   if (!b) return SCFT_E_ARG;
-  if (w)
+  if (w) {
+    touch_pages(w, sizeof(double) * b->total_u);
     HIPCHK(hipMemcpyAsync(w, b->d_w, sizeof(double) * b->total_u, hipMemcpyDeviceToHost,
                           b->stream));
+  }
   std::vector<int> it(b->n_inst, 0);
   std::vector<unsigned> stv(b->n_inst, 0);
   if (b->d_iters)
@@ -1368,6 +1426,7 @@ scft_batch* g_one = nullptr;  // single-instance context of the drop-in entries
 int g_one_n = -1;
 std::vector<double> g_target;  // from scft_set_target (all nodes)
 std::vector<double> g_x, g_ptall, g_ptu, g_r;
+std::vector<double> g_pt_resident;  // the target that g_one's device copy holds
 int g_last_status = SCFT_OK;
 }  // namespace
 
@@ -1400,6 +1459,7 @@ static int init_locked(const scft_config* cfg) {
   if (g_one) scft_batch_destroy(g_one);
   g_one = nullptr;
   g_one_n = -1;
+  g_pt_resident.clear();
   g_init = true;
   return SCFT_OK;
 }
@@ -1454,6 +1514,7 @@ static int dropin_eval(int n, const double* w, double* r) {
   if (g_one_n != n) {
     if (g_one) scft_batch_destroy(g_one);
     g_one = nullptr;
+    g_pt_resident.clear();
     g_x.assign(M, 0.0);
     mesh_uniform(M, g_cfg.L, g_x.data());
     g_ptu.assign(n, 1.0);
@@ -1483,7 +1544,11 @@ static int dropin_eval(int n, const double* w, double* r) {
     target_position(M, g_x.data(), g_cfg.tau, dd, g_ptall.data());
   }
   for (int u = 0; u < n; u++) g_ptu[u] = g_ptall[u + 1];
-  SCFT_TRY(batch_set_target(g_one, g_ptu.data()));
+  if (g_pt_resident != g_ptu) {  // (compared by value: callers change it in place)
+    g_pt_resident.clear();
+    SCFT_TRY(batch_set_target(g_one, g_ptu.data()));
+    g_pt_resident = g_ptu;
+  }
   // the consistent w-mass reads the field at the walls: extrapolated from the
   // unknowns by a natural spline as the deal.II evaluator does (DD: both
   // walls; DN: the wall at x = 0; a single unknown keeps zero walls)

@@ -489,12 +489,7 @@ __global__ void __launch_bounds__(64 * W) irk4_kernel(MarchArgs a) {
   extern __shared__ double pw_lds[];
   const int tid = threadIdx.x;
   double* slab = a.slabs + (long long)blockIdx.x * a.slab_stride;
-  for (;;) {
-    if (tid == 0) s_next = atomicAdd(a.queue, 1);
-    wg_barrier();
-    const int it = __builtin_amdgcn_readfirstlane(s_next);
-    wg_barrier();
-    if (it >= a.n_items) break;
+  for (int it = blockIdx.x; it < a.n_items; it = next_item(a, tid, &s_next)) {
     const int inst = __builtin_amdgcn_readfirstlane(a.items[it]);
     const unsigned st = __builtin_amdgcn_readfirstlane(a.status[inst]);
     if (st & ST_DONE_MASK) continue;

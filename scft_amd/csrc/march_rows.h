@@ -6,6 +6,21 @@
 
 namespace scft {
 
+// The persistent workgroups' next item: its own number first (the caller's
+// loop), then from the launch's counter, which is not read when the grid covers
+// all items.  Thread 0 takes the index and broadcasts it through LDS; the value
+// is workgroup-uniform, so every wave leaves the loop together.  The two
+// barriers also separate an instance's use of LDS from the next one's.
+__device__ __forceinline__ int next_item(const MarchArgs& a, int tid, int* s_next) {
+  const int grid = static_cast<int>(gridDim.x);
+  if (a.n_items <= grid) return a.n_items;
+  if (tid == 0) *s_next = grid + atomicAdd(a.queue, 1);
+  wg_barrier();
+  const int it = __builtin_amdgcn_readfirstlane(*s_next);
+  wg_barrier();  // everyone has read it before thread 0 overwrites it
+  return it;
+}
+
 template <int W>
 struct MarchShared {
   // forward, then backward wave totals (per step, two sets in turn), and a

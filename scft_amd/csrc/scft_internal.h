@@ -36,7 +36,7 @@ struct MarchArgs {
   double* slabs;          // q-slab scratch, one region per workgroup
   long long slab_stride;  // doubles per workgroup region (N_max/2 slabs)
   const int* items;       // instance ids of this bucket, largest first
-  int* queue;             // next item to take (zeroed before every launch)
+  int* queue;             // items taken past the grid's first (zeroed before a launch of more)
   int n_items;
   int half_max;           // largest N/2 of the bucket (IRK4: LDS weight table size - 1)
   int seg;                // 1: every slab is kept, MARCH_SEG: every MARCH_SEG-th (march.hip)
