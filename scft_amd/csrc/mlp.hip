@@ -5,16 +5,17 @@
 // oracle/oracle_mlp.c packs them: per layer W (dout x din, row-major), then
 // b (dout).
 //
-// Every product is one kernel, `gemm_kernel`: C[m][n] = sum_k A(m,k) B(k,n)
-// with arbitrary element strides for A and B, FP32 operands and FP32
-// accumulation on the matrix cores (v_mfma_f32_16x16x4f32), and a fused
-// epilogue (bias + tanh for hidden layers, bias for the output layer, the
-// tanh derivative for back-propagated deltas, or nothing).  Workgroups of 4
-// waves own a 32 x 32 tile of C, each wave one 16 x 16 block; K advances in
-// chunks of 64 staged in LDS, each operand loaded along whichever of its
-// strides is 1.  The training products are 256 x 256 x 256 at batch 256:
-// small tiles give 64 workgroups for them, and deep chunks four round trips
-// to memory per tile instead of sixteen.
+// Networks whose activations of 16 rows fit in LDS run whole: one launch takes
+// the rows through all layers (in training also through the loss and the
+// deltas), one makes all gradients and the Adam step (net_kernel,
+// grad_kernel).  Wider or deeper ones go product by product: `gemm_kernel` is
+// C[m][n] = sum_k A(m,k) B(k,n) with arbitrary element strides for A and B,
+// FP32 operands and FP32 accumulation on the matrix cores
+// (v_mfma_f32_16x16x4f32), and a fused epilogue (bias + tanh for hidden
+// layers, bias for the output layer, the tanh derivative for back-propagated
+// deltas, or nothing).  Workgroups of 4 waves own a 32 x 32 tile of C, each
+// wave one 16 x 16 block; K advances in chunks of 64 staged in LDS, each
+// operand loaded along whichever of its strides is 1.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -143,18 +144,26 @@ __global__ void mse_kernel(const float* __restrict__ y, const float* __restrict_
 }
 
 // Adam (Kingma & Ba 2015, Algorithm 1) with bias corrections c1, c2
-__global__ void adam_kernel(long long n, float* __restrict__ p, const float* __restrict__ g,
-                            float* __restrict__ m, float* __restrict__ v, float lr, float b1,
-                            float b2, float eps, float c1, float c2) {
+struct AdamArgs {
+  float *p, *m, *v;
+  float lr, b1, b2, eps, c1, c2;
+};
+
+__device__ __forceinline__ float adam_update(const AdamArgs& a, long long k, float gk, float pk,
+                                             float mo, float vo) {
+  const float mk = a.b1 * mo + (1.f - a.b1) * gk;
+  const float vk = a.b2 * vo + (1.f - a.b2) * gk * gk;
+  a.m[k] = mk;
+  a.v[k] = vk;
+  const float pn = pk - a.lr * (mk / a.c1) / (sqrtf(vk / a.c2) + a.eps);
+  a.p[k] = pn;
+  return pn;
+}
+
+__global__ void adam_kernel(long long n, const float* __restrict__ g, AdamArgs a) {
   for (long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x; k < n;
-       k += (long long)gridDim.x * blockDim.x) {
-    const float gk = g[k];
-    const float mk = b1 * m[k] + (1.f - b1) * gk;
-    const float vk = b2 * v[k] + (1.f - b2) * gk * gk;
-    m[k] = mk;
-    v[k] = vk;
-    p[k] -= lr * (mk / c1) / (sqrtf(vk / c2) + eps);
-  }
+       k += (long long)gridDim.x * blockDim.x)
+    adam_update(a, k, g[k], a.p[k], a.m[k], a.v[k]);
 }
 
 // rows idx[0..batch) of src (row length len) into dst
@@ -166,6 +175,337 @@ __global__ void gather_kernel(const float* __restrict__ src, const int* __restri
     const long long b = k / len, c = k % len;
     dst[k] = src[(long long)idx[b] * len + c];
   }
+}
+
+// ------------------------------------------------------- whole networks
+// The rows of a batch are independent up to the weight gradients, so one
+// launch takes 16 rows per workgroup through all layers, and in training on
+// through the loss and the deltas of every layer, with the activations in LDS:
+// a launch per product spent 13-21 us each on 64 workgroups and four memory
+// round trips, for 0.5 us of matrix work.
+//
+// The weights are read in the order of the matrix instruction's operand: tile
+// (output block n, input block j) holds, for lane l and element e,
+// W(16 n + l % 16, 16 j + 4 e + l / 16): one 16-byte load per lane feeds four
+// instructions, and the products are summed in ascending k as gemm_kernel
+// does (same bits).  A second copy holds the transpose for the deltas.  Both
+// are written with the parameters.  A row of tiles is padded to kRing blocks,
+// the loads that a wave keeps in flight: 16 waves x 8 KB cover the latency of
+// L2, and the next tile's loads start before the barrier between layers.
+//
+// Bound by the matrix instructions of the 16 compute units that a batch of 256
+// occupies (27 us at 2.4 GHz of the 50 us that 133 - 4 x 256 - 136 takes there,
+// forward and deltas; the rest is the barrier and the result of each of the
+// nine products).  16 rows are the instruction's least, so a batch of 256
+// cannot use more units; rows split over units would meet at every layer.
+// With grad_kernel's 12 us a step takes 62 us, 322 us in 23 launches before;
+// a forward pass of 592 rows 100 -> 28 us.
+constexpr int ROWS = 16;       // rows of a workgroup
+constexpr int NET_WAVES = 16;  // waves of a workgroup, one 16-column tile each at a time
+static_assert(NET_WAVES == ROWS && NET_WAVES >= 8, "a wave stages a row, and a layer's bias");
+constexpr int kRing = 8;
+constexpr int kMaxLayers = 8;
+constexpr int kMaxLds = 150 * 1024;
+
+inline int blocks16(int n) { return (n + 15) / 16; }
+inline long long packed_size(int dout, int din) {  // floats
+  return (long long)blocks16(dout) * ((blocks16(din) + kRing - 1) / kRing * kRing) * 256;
+}
+
+struct NetPhase {      // one product: forward layer l, then the deltas of layer l
+  const float* w;      // packed tiles
+  const float* bias;   // forward
+  float* out;          // global copy of the result (nullptr: none)
+  int J, NB;           // blocks of 16 along the sum and along the outputs
+  int cols;            // outputs
+  int in, dst, act;    // LDS offsets (floats): input, result; bias or activation (deltas)
+};
+
+struct NetArgs {
+  int L, phases, batch, din, lds0;
+  const float* x;      // input rows
+  const int* idx;      // nullptr: row b is x + b * din, else x + idx[b] * din
+  float* x_out;        // training: the gathered rows
+  const float* t;      // training: targets, indexed as x
+  float scale;         // delta = scale (y - t)
+  double* loss;
+  NetPhase ph[2 * kMaxLayers - 1];
+};
+
+__device__ __forceinline__ floatx4 mfma4(float4 a, float4 b, floatx4 acc) {
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, acc, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, acc, 0, 0, 0);
+}
+
+template <bool TRAIN>
+__global__ void __launch_bounds__(64 * NET_WAVES) net_kernel(NetArgs g) {
+  extern __shared__ __align__(16) float lds[];
+  __shared__ double red[NET_WAVES];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, q = lane >> 4;
+  const int row0 = blockIdx.x * ROWS;
+
+  auto tile_row = [&](int ph, int nb) {
+    const int jp = (g.ph[ph].J + kRing - 1) / kRing * kRing;
+    return reinterpret_cast<const float4*>(g.ph[ph].w) + (size_t)nb * jp * 64 + lane;
+  };
+  // the wave's first tile of a phase at or after `ph`
+  int ph_w = 0;
+  while (ph_w < g.phases && wave >= g.ph[ph_w].NB) ph_w++;
+  const float4* w = tile_row(ph_w < g.phases ? ph_w : 0, ph_w < g.phases ? wave : 0);
+  float4 ring[kRing];
+#pragma unroll
+  for (int e = 0; e < kRing; e++) ring[e] = w[e * 64];
+
+  // Input rows, targets (where their deltas will be) and biases to LDS: wave v
+  // loads row v and the bias of layer v, all loads of 256 columns before the
+  // first use.  Rows with k = 16 j + 4 e + q at 16 j + 4 q + e, zeros outside.
+  {
+    const NetPhase& last = g.ph[g.L - 1];
+    const NetPhase& mine = g.ph[min(wave, g.L - 1)];
+    const int cx = g.ph[0].J * 16, ct = TRAIN ? last.NB * 16 : 0;
+    const int cb = wave < g.L ? mine.NB * 16 : 0;
+    const int row = row0 + wave;
+    const bool live = row < g.batch;
+    const long long src = !live ? 0 : g.idx ? g.idx[row] : row;
+    const float* px = g.x + src * g.din;
+    const float* pt = TRAIN ? g.t + src * last.cols : nullptr;
+    for (int k0 = 0; k0 < max(max(cx, ct), cb); k0 += 256) {
+      float x[4], t[4], b[4];
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const int k = k0 + 64 * c + lane;
+        x[c] = t[c] = b[c] = 0.f;
+        if (k < cb && k < mine.cols) b[c] = mine.bias[k];
+        if (live && k < g.din) x[c] = px[k];
+        if (TRAIN && live && k < last.cols) t[c] = pt[k];
+      }
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const int k = k0 + 64 * c + lane, pos = (k & ~15) + 4 * (k & 3) + ((k >> 2) & 3);
+        if (k < cb) lds[mine.act + k] = b[c];
+        if (k < cx) lds[g.lds0 + wave * (cx + 4) + pos] = x[c];
+        if (k < ct) lds[last.dst + wave * (ct + 4) + pos] = t[c];
+        if (TRAIN && live && k < g.din) g.x_out[(long long)row * g.din + k] = x[c];
+      }
+    }
+  }
+  __syncthreads();
+
+  double sq = 0.0;
+  for (int ph = 0; ph < g.phases; ph++) {
+    const NetPhase& f = g.ph[ph];
+    const int J = f.J, SA = J * 16 + 4, SO = f.NB * 16 + 4;
+    const float4* a = reinterpret_cast<const float4*>(lds + f.in + r * SA + 4 * q);
+    for (int nb = wave; nb < f.NB; nb += NET_WAVES) {
+      const float4* next = w;  // (no tile left: any)
+      if (nb + NET_WAVES < f.NB) {
+        next = tile_row(ph, nb + NET_WAVES);
+      } else {
+        int p2 = ph + 1;
+        while (p2 < g.phases && wave >= g.ph[p2].NB) p2++;
+        if (p2 < g.phases) next = tile_row(p2, wave);
+      }
+      floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
+      int j0 = 0;
+      float4 av[2] = {a[0], a[min(1, J - 1) * 4]};
+      for (; j0 + kRing <= J; j0 += kRing) {
+        const float4* nx = j0 + kRing < J ? w + (j0 + kRing) * 64 : next;
+#pragma unroll
+        for (int e = 0; e < kRing; e++) {
+          acc = mfma4(av[e & 1], ring[e], acc);
+          // after their use: the same registers; and not moved to the group's
+          // end, where the scheduler would put them
+          ring[e] = nx[e * 64];
+          av[e & 1] = a[min(j0 + e + 2, J - 1) * 4];
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      if (j0 < J) {  // the last, partly filled group
+#pragma unroll
+        for (int e = 0; e < kRing; e++) {
+          if (j0 + e < J) {
+            acc = mfma4(av[e & 1], ring[e], acc);
+            av[e & 1] = a[min(j0 + e + 2, J - 1) * 4];
+          }
+          ring[e] = next[e * 64];
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      w = next;
+      // lane holds rows 4 q + e of column n; what the result needs is in LDS: a
+      // wait for a load from memory would be one for the ring's, too
+      const int n = nb * 16 + r;
+      const bool in = n < f.cols;
+      const float bias = ph < g.L ? lds[f.act + n] : 0.f;
+      const int pos = nb * 16 + 4 * (r & 3) + (r >> 2);
+      float* o = lds + f.dst + 4 * q * SO + pos;  // rows 4 q + e: every SO
+      const int live = in ? g.batch - row0 - 4 * q : 0;  // rows of the four in the batch
+      float v[4];
+      if (ph < g.L) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = acc[e] + bias;
+        if (ph < g.L - 1) {
+#pragma unroll
+          for (int e = 0; e < 4; e++) v[e] = tanhf(v[e]);
+        } else if (TRAIN) {
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const float err = e < live ? v[e] - o[e * SO] : 0.f;  // o: the target
+            v[e] = g.scale * err;
+            sq += (double)err * err;
+          }
+        }
+      } else {
+        const float* act = lds + f.act + 4 * q * SO + pos;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const float y = act[e * SO];
+          v[e] = acc[e] * (1.f - y * y);
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; e++) o[e * SO] = in ? v[e] : 0.f;
+      if (f.out) {
+        float* out = f.out + (long long)(row0 + 4 * q) * f.cols + n;
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          if (e < live) out[(long long)e * f.cols] = v[e];
+      }
+    }
+    __syncthreads();
+  }
+  if (TRAIN) {
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) sq += __shfl_xor(sq, off);
+    if (lane == 0) red[wave] = sq;
+    __syncthreads();
+    if (tid == 0) {
+      double tot = 0.0;
+      for (int v = 0; v < NET_WAVES; v++) tot += red[v];
+      atomicAdd(g.loss, tot);
+    }
+  }
+}
+
+// The two packed copies of one weight (o, i); `jf`, `jb`: padded blocks of a
+// row of tiles.
+__device__ __forceinline__ void store_packed(float* wf, float* wb, int jf, int jb, int o, int i,
+                                             float v) {
+  wf[((long long)(o >> 4) * jf + (i >> 4)) * 256 + ((i & 3) * 16 + (o & 15)) * 4 +
+     ((i >> 2) & 3)] = v;
+  wb[((long long)(i >> 4) * jb + (o >> 4)) * 256 + ((o & 3) * 16 + (i & 15)) * 4 +
+     ((o >> 2) & 3)] = v;
+}
+
+struct GradLayer {
+  const float *delta, *act;  // batch x dout, batch x din
+  float *wf, *wb;            // packed copies
+  long long off;             // of the layer's parameters
+  int dout, din, jf, jb, tile0, tiles_n;
+};
+
+struct GradArgs {
+  int L, batch;
+  float* g;
+  AdamArgs adam;
+  GradLayer l[kMaxLayers];
+};
+
+// All layers' weight and bias gradients of a batch, and with ADAM the step
+// itself: a workgroup takes a 32 x 32 tile of one layer's weights, a wave a
+// 16 x 16 block; both operands are contiguous along the block's rows or
+// columns, so they go from L2 to the matrix cores without LDS, 16 steps of
+// the sum in flight.  The bias gradient is the running sum of the operand
+// that the lane loads anyway, in the order of colsum_kernel (rows b = q mod
+// 4, then the four parts), the sum over the batch that of gemm_kernel.
+template <bool ADAM>
+__global__ void __launch_bounds__(256) grad_kernel(GradArgs g) {
+  constexpr int G = 16;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int li = 0;
+  while (li + 1 < g.L && (int)blockIdx.x >= g.l[li + 1].tile0) li++;
+  const GradLayer& l = g.l[li];
+  const int tile = blockIdx.x - l.tile0;
+  const int o0 = (tile / l.tiles_n) * 32 + (wave >> 1) * 16;
+  const int i0 = (tile % l.tiles_n) * 32 + (wave & 1) * 16;
+  if (o0 >= l.dout || i0 >= l.din) return;
+  const int r = lane & 15, q = lane >> 4;
+  // columns outside the layer repeat its last one; their results are dropped
+  const float* pa = l.delta + min(o0 + r, l.dout - 1);
+  const float* pb = l.act + min(i0 + r, l.din - 1);
+  const int i = i0 + r, ob = o0 + 4 * q;  // the lane's column and first row of the result
+  float po[4], mo[4], vo[4];
+  if (ADAM) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const long long k = l.off + (long long)min(ob + e, l.dout - 1) * l.din + min(i, l.din - 1);
+      po[e] = g.adam.p[k];
+      mo[e] = g.adam.m[k];
+      vo[e] = g.adam.v[k];
+    }
+  }
+  floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
+  float sum = 0.f;
+  auto load = [&](int b0, float (&a)[G], float (&b)[G]) {
+#pragma unroll
+    for (int s = 0; s < G; s++) {  // rows past the batch: zeros
+      const int row = b0 + 4 * s + q, rc = min(row, g.batch - 1);
+      a[s] = pa[(long long)rc * l.dout];
+      b[s] = pb[(long long)rc * l.din];
+      if (row >= g.batch) a[s] = b[s] = 0.f;
+    }
+  };
+  float a[G], b[G], a2[G], b2[G];
+  load(0, a, b);
+  for (int b0 = 0; b0 < g.batch; b0 += 4 * G) {
+    if (b0 + 4 * G < g.batch) load(b0 + 4 * G, a2, b2);
+#pragma unroll
+    for (int s = 0; s < G; s++) {
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], acc, 0, 0, 0);
+      sum += a[s];
+    }
+#pragma unroll
+    for (int s = 0; s < G; s++) {
+      a[s] = a2[s];
+      b[s] = b2[s];
+    }
+  }
+  if (i < l.din) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      if (ob + e >= l.dout) continue;
+      const long long k = l.off + (long long)(ob + e) * l.din + i;
+      g.g[k] = acc[e];
+      if (ADAM) {
+        const float pn = adam_update(g.adam, k, acc[e], po[e], mo[e], vo[e]);
+        store_packed(l.wf, l.wb, l.jf, l.jb, ob + e, i, pn);
+      }
+    }
+  }
+  if (i0 == 0) {
+    sum += __shfl_xor(sum, 16);
+    sum += __shfl_xor(sum, 32);
+    const int o = o0 + r;
+    if (q == 0 && o < l.dout) {
+      const long long k = l.off + (long long)l.dout * l.din + o;
+      g.g[k] = sum;
+      if (ADAM) adam_update(g.adam, k, sum, g.adam.p[k], g.adam.m[k], g.adam.v[k]);
+    }
+  }
+}
+
+// the packed copies of one layer's weights, after the parameters were set
+__global__ void pack_kernel(const float* __restrict__ W, int dout, int din, int jf, int jb,
+                            float* __restrict__ wf, float* __restrict__ wb) {
+  const long long n = (long long)dout * din;
+  for (long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x; k < n;
+       k += (long long)gridDim.x * blockDim.x)
+    store_packed(wf, wb, jf, jb, (int)(k / din), (int)(k % din), W[k]);
 }
 
 }  // namespace
@@ -182,6 +522,12 @@ struct scft_mlp {
   float *d_p = nullptr, *d_g = nullptr, *d_m = nullptr, *d_v = nullptr;
   std::vector<float*> d_act;       // L + 1 activation buffers [cap_batch x dims[l]]
   float *d_delta0 = nullptr, *d_delta1 = nullptr, *d_t = nullptr;
+  // networks that net_kernel takes: packed weights, deltas of every layer
+  bool whole = false;
+  int lds_fwd = 0, lds_train = 0;  // bytes
+  float* d_pack = nullptr;
+  std::vector<long long> pack_f, pack_b;  // offsets in d_pack
+  std::vector<float*> d_delta;
   double* d_loss = nullptr;
   int adam_t = 0;
   hipStream_t stream = nullptr;
@@ -205,23 +551,167 @@ int mlp_dalloc(float** p, long long n) {
              : SCFT_E_NOMEM;
 }
 
-int ensure_batch(scft_mlp* m, int batch) {
-  if (batch <= m->cap_batch) return SCFT_OK;
+void free_batch(scft_mlp* m) {
   for (auto p : m->d_act) (void)hipFree(p);
+  for (auto p : m->d_delta) (void)hipFree(p);
   (void)hipFree(m->d_delta0);
   (void)hipFree(m->d_delta1);
   (void)hipFree(m->d_t);
   m->d_act.assign(m->dims.size(), nullptr);
+  m->d_delta.assign(m->dims.size() - 1, nullptr);
+  m->d_delta0 = m->d_delta1 = m->d_t = nullptr;
+  m->cap_batch = 0;
+}
+
+int ensure_batch(scft_mlp* m, int batch) {
+  if (batch <= m->cap_batch) return SCFT_OK;
+  free_batch(m);
   int widest = 0;
   for (size_t l = 0; l < m->dims.size(); l++) {
     if (mlp_dalloc(&m->d_act[l], (long long)batch * m->dims[l])) return SCFT_E_NOMEM;
     widest = std::max(widest, m->dims[l]);
+    if (m->whole && l > 0 && mlp_dalloc(&m->d_delta[l - 1], (long long)batch * m->dims[l]))
+      return SCFT_E_NOMEM;
   }
-  if (mlp_dalloc(&m->d_delta0, (long long)batch * widest) ||
-      mlp_dalloc(&m->d_delta1, (long long)batch * widest) ||
-      mlp_dalloc(&m->d_t, (long long)batch * m->dims.back()))
+  if (!m->whole && (mlp_dalloc(&m->d_delta0, (long long)batch * widest) ||
+                    mlp_dalloc(&m->d_delta1, (long long)batch * widest)))
     return SCFT_E_NOMEM;
+  if (mlp_dalloc(&m->d_t, (long long)batch * m->dims.back())) return SCFT_E_NOMEM;
   m->cap_batch = batch;
+  return SCFT_OK;
+}
+
+int ring16(int n) { return (blocks16(n) + kRing - 1) / kRing * kRing; }
+
+// net_kernel takes networks of at most kMaxLayers layers whose activations of
+// 16 rows fit in LDS beside two buffers for the running input and delta; the
+// default shape (133, 4 x 256, 136) needs 102 KB.  Others go layer by layer.
+void plan_whole(scft_mlp* m) {
+  const int L = static_cast<int>(m->dims.size()) - 1;
+  long long hidden = 0, bias = 0;
+  int widest = 0;
+  for (int l = 0; l <= L; l++) {
+    const int row = blocks16(m->dims[l]) * 16 + 4;
+    widest = std::max(widest, row);
+    if (l > 0 && l < L) hidden += row;
+    if (l > 0) bias += row - 4;
+  }
+  const long long fwd = (long long)sizeof(float) * (ROWS * 2 * widest + bias);
+  const long long train = fwd + (long long)sizeof(float) * ROWS * hidden;
+  m->whole = L <= kMaxLayers && train <= kMaxLds;
+  m->lds_fwd = m->whole ? static_cast<int>(fwd) : 0;
+  m->lds_train = m->whole ? static_cast<int>(train) : 0;
+}
+
+int pack(scft_mlp* m) {
+  if (!m->whole) return SCFT_OK;
+  for (size_t l = 0; l + 1 < m->dims.size(); l++) {
+    const int din = m->dims[l], dout = m->dims[l + 1];
+    hipLaunchKernelGGL(pack_kernel, dim3(64), dim3(256), 0, m->stream, m->d_p + m->off[l], dout,
+                       din, ring16(din), ring16(dout), m->d_pack + m->pack_f[l],
+                       m->d_pack + m->pack_b[l]);
+    MLPCHK(hipGetLastError());
+  }
+  return SCFT_OK;
+}
+
+// `batch` rows of x (idx: gathered) through the network; t == nullptr: the
+// outputs into d_act.back(), else the loss onto *d_loss and every layer's
+// input and delta into d_act and d_delta.
+int run_net(scft_mlp* m, int batch, const float* x, const float* t, const int* idx) {
+  const int L = static_cast<int>(m->dims.size()) - 1;
+  NetArgs g{};
+  g.L = L;
+  g.phases = t ? 2 * L - 1 : L;
+  g.batch = batch;
+  g.din = m->dims[0];
+  g.x = x;
+  g.idx = idx;
+  g.x_out = t ? m->d_act[0] : nullptr;
+  g.t = t;
+  g.scale = 2.f / static_cast<float>((long long)batch * m->dims[L]);
+  g.loss = m->d_loss;
+  int widest = 0;
+  for (int d : m->dims) widest = std::max(widest, blocks16(d) * 16 + 4);
+  const int buf[2] = {0, ROWS * widest};  // the inputs go to buf[0]
+  int act[kMaxLayers];                    // LDS offset of d_act[l]
+  act[0] = buf[0];
+  int lds = 2 * ROWS * widest;
+  for (int l = 0; l < L; l++) {
+    g.ph[l].act = lds;
+    lds += blocks16(m->dims[l + 1]) * 16;
+  }
+  for (int l = 1; l < L; l++) {
+    act[l] = t ? lds : buf[l & 1];
+    lds += ROWS * (blocks16(m->dims[l]) * 16 + 4);
+  }
+  g.lds0 = act[0];
+  for (int l = 0; l < L; l++) {
+    NetPhase& f = g.ph[l];
+    f.w = m->d_pack + m->pack_f[l];
+    f.bias = m->d_p + m->off[l] + (long long)m->dims[l + 1] * m->dims[l];
+    f.cols = m->dims[l + 1];
+    f.J = blocks16(m->dims[l]);
+    f.NB = blocks16(f.cols);
+    f.in = act[l];
+    f.dst = l + 1 < L ? act[l + 1] : t ? buf[1] : buf[L & 1];
+    f.out = t ? (l + 1 < L ? m->d_act[l + 1] : m->d_delta[l]) : l + 1 < L ? nullptr : m->d_act[L];
+  }
+  for (int l = L - 1, ph = L, k = 1; t && l > 0; l--, ph++, k ^= 1) {  // deltas of layer l - 1
+    NetPhase& f = g.ph[ph];
+    f.w = m->d_pack + m->pack_b[l];
+    f.cols = m->dims[l];
+    f.J = blocks16(m->dims[l + 1]);
+    f.NB = blocks16(f.cols);
+    f.in = buf[k];
+    f.dst = buf[k ^ 1];
+    f.act = act[l];
+    f.out = m->d_delta[l - 1];
+  }
+  const dim3 grid((batch + ROWS - 1) / ROWS), block(64 * NET_WAVES);
+  if (t)
+    hipLaunchKernelGGL(net_kernel<true>, grid, block, m->lds_train, m->stream, g);
+  else
+    hipLaunchKernelGGL(net_kernel<false>, grid, block, m->lds_fwd, m->stream, g);
+  MLPCHK(hipGetLastError());
+  return SCFT_OK;
+}
+
+AdamArgs adam_args(const scft_mlp* m, float lr) {
+  const float b1 = 0.9f, b2 = 0.999f;
+  const float c1 = 1.f - std::pow(b1, (float)m->adam_t);
+  const float c2 = 1.f - std::pow(b2, (float)m->adam_t);
+  return AdamArgs{m->d_p, m->d_m, m->d_v, lr, b1, b2, 1e-8f, c1, c2};
+}
+
+// the gradients of the batch that run_net left, and with `adam` the step
+int run_grad(scft_mlp* m, int batch, const AdamArgs* adam) {
+  GradArgs g{};
+  g.L = static_cast<int>(m->dims.size()) - 1;
+  g.batch = batch;
+  g.g = m->d_g;
+  if (adam) g.adam = *adam;
+  int tiles = 0;
+  for (int l = 0; l < g.L; l++) {
+    GradLayer& a = g.l[l];
+    a.delta = m->d_delta[l];
+    a.act = m->d_act[l];
+    a.wf = m->d_pack + m->pack_f[l];
+    a.wb = m->d_pack + m->pack_b[l];
+    a.off = m->off[l];
+    a.din = m->dims[l];
+    a.dout = m->dims[l + 1];
+    a.jf = ring16(a.din);
+    a.jb = ring16(a.dout);
+    a.tile0 = tiles;
+    a.tiles_n = (a.din + 31) / 32;
+    tiles += a.tiles_n * ((a.dout + 31) / 32);
+  }
+  if (adam)
+    hipLaunchKernelGGL(grad_kernel<true>, dim3(tiles), dim3(256), 0, m->stream, g);
+  else
+    hipLaunchKernelGGL(grad_kernel<false>, dim3(tiles), dim3(256), 0, m->stream, g);
+  MLPCHK(hipGetLastError());
   return SCFT_OK;
 }
 
@@ -234,7 +724,8 @@ hipError_t gemm(hipStream_t s, const float* A, long long a_m, long long a_k, con
   return hipGetLastError();
 }
 
-// forward of `batch` rows already in d_act[0]; activations kept for backward
+// forward of `batch` rows already in d_act[0], layer by layer; activations kept
+// for backward
 int forward(scft_mlp* m, int batch) {
   const int L = static_cast<int>(m->dims.size()) - 1;
   for (int l = 0; l < L; l++) {
@@ -313,6 +804,14 @@ extern "C" int scft_mlp_create(scft_mlp** out, int n_layers, const int* dims,
   }
   m->off[n_layers] = o;
   m->n_params = o;
+  plan_whole(m);
+  long long np = 0;
+  for (int l = 0; l < n_layers && m->whole; l++) {
+    m->pack_f.push_back(np);
+    np += packed_size(dims[l + 1], dims[l]);
+    m->pack_b.push_back(np);
+    np += packed_size(dims[l], dims[l + 1]);
+  }
   // Glorot-uniform weights, zero biases, from splitmix64(seed)
   std::vector<float> p(o, 0.f);
   uint64_t s = seed;
@@ -325,16 +824,24 @@ extern "C" int scft_mlp_create(scft_mlp** out, int n_layers, const int* dims,
   }
   if (hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) != hipSuccess ||
       mlp_dalloc(&m->d_p, o) || mlp_dalloc(&m->d_g, o) || mlp_dalloc(&m->d_m, o) ||
-      mlp_dalloc(&m->d_v, o) ||
+      mlp_dalloc(&m->d_v, o) || mlp_dalloc(&m->d_pack, np) ||
       hipMalloc(reinterpret_cast<void**>(&m->d_loss), sizeof(double)) != hipSuccess) {
     delete m;
     return SCFT_E_NOMEM;
   }
   if (hipMemcpy(m->d_p, p.data(), sizeof(float) * o, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemset(m->d_m, 0, sizeof(float) * o) != hipSuccess ||
-      hipMemset(m->d_v, 0, sizeof(float) * o) != hipSuccess) {
+      hipMemset(m->d_v, 0, sizeof(float) * o) != hipSuccess ||
+      (np > 0 && hipMemset(m->d_pack, 0, sizeof(float) * np) != hipSuccess) ||
+      hipStreamSynchronize(nullptr) != hipSuccess || pack(m)) {
     delete m;
     return SCFT_E_HIP;
+  }
+  if (m->whole) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(net_kernel<true>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(net_kernel<false>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
   }
   *out = m;
   return SCFT_OK;
@@ -343,10 +850,8 @@ extern "C" int scft_mlp_create(scft_mlp** out, int n_layers, const int* dims,
 extern "C" int scft_mlp_destroy(scft_mlp* m) {
   if (!m) return SCFT_OK;
   (void)hipStreamSynchronize(m->stream);
-  for (auto p : m->d_act) (void)hipFree(p);
-  (void)hipFree(m->d_delta0);
-  (void)hipFree(m->d_delta1);
-  (void)hipFree(m->d_t);
+  free_batch(m);
+  (void)hipFree(m->d_pack);
   (void)hipFree(m->d_p);
   (void)hipFree(m->d_g);
   (void)hipFree(m->d_m);
@@ -377,6 +882,8 @@ extern "C" int scft_mlp_set_params(scft_mlp* m, const float* in) {
   MLPCHK(hipMemset(m->d_m, 0, sizeof(float) * m->n_params));
   MLPCHK(hipMemset(m->d_v, 0, sizeof(float) * m->n_params));
   m->adam_t = 0;
+  MLPCHK(hipStreamSynchronize(nullptr));
+  if (int rc = pack(m)) return rc;
   return SCFT_OK;
 }
 
@@ -409,7 +916,8 @@ extern "C" int scft_mlp_forward(scft_mlp* m, int batch, const float* X, float* Y
   normalise_rows(m, X, batch, xn);
   MLPCHK(hipMemcpyAsync(m->d_act[0], xn.data(), sizeof(float) * xn.size(),
                         hipMemcpyHostToDevice, m->stream));
-  if (int rc = forward(m, batch)) return rc;
+  if (int rc = m->whole ? run_net(m, batch, m->d_act[0], nullptr, nullptr) : forward(m, batch))
+    return rc;
   const int dout = m->dims.back();
   MLPCHK(hipMemcpyAsync(Y, m->d_act.back(), sizeof(float) * (size_t)batch * dout,
                         hipMemcpyDeviceToHost, m->stream));
@@ -427,9 +935,13 @@ int scft_mlp_forward_resident(scft_mlp* m, int batch, const float* d_xn, const f
   if (!m || batch < 1 || !d_xn || !d_out) return SCFT_E_ARG;
   if (int rc = ensure_batch(m, batch)) return rc;
   const int din = m->dims.front();
-  MLPCHK(hipMemcpyAsync(m->d_act[0], d_xn, sizeof(float) * (size_t)batch * din,
-                        hipMemcpyDeviceToDevice, m->stream));
-  if (int rc = forward(m, batch)) return rc;
+  if (m->whole) {
+    if (int rc = run_net(m, batch, d_xn, nullptr, nullptr)) return rc;
+  } else {
+    MLPCHK(hipMemcpyAsync(m->d_act[0], d_xn, sizeof(float) * (size_t)batch * din,
+                          hipMemcpyDeviceToDevice, m->stream));
+    if (int rc = forward(m, batch)) return rc;
+  }
   MLPCHK(hipStreamSynchronize(m->stream));
   *d_out = m->d_act.back();
   if (ym) *ym = m->ym.empty() ? nullptr : m->ym.data();
@@ -459,8 +971,14 @@ extern "C" int scft_mlp_loss_grad(scft_mlp* m, int batch, const float* X, const 
                         hipMemcpyHostToDevice, m->stream));
   MLPCHK(hipMemcpyAsync(m->d_t, T, sizeof(float) * (size_t)batch * dout, hipMemcpyHostToDevice,
                         m->stream));
-  if (int rc = forward(m, batch)) return rc;
-  if (int rc = backward(m, batch)) return rc;
+  if (m->whole) {
+    MLPCHK(hipMemsetAsync(m->d_loss, 0, sizeof(double), m->stream));
+    if (int rc = run_net(m, batch, m->d_act[0], m->d_t, nullptr)) return rc;
+    if (int rc = run_grad(m, batch, nullptr)) return rc;
+  } else {
+    if (int rc = forward(m, batch)) return rc;
+    if (int rc = backward(m, batch)) return rc;
+  }
   double l = 0.0;
   MLPCHK(hipMemcpyAsync(&l, m->d_loss, sizeof(double), hipMemcpyDeviceToHost, m->stream));
   if (grad)
@@ -474,13 +992,11 @@ extern "C" int scft_mlp_loss_grad(scft_mlp* m, int batch, const float* X, const 
 // One Adam step on the gradient currently held (after scft_mlp_loss_grad).
 extern "C" int scft_mlp_adam_step(scft_mlp* m, float lr) {
   if (!m) return SCFT_E_ARG;
-  const float b1 = 0.9f, b2 = 0.999f;
   m->adam_t++;
-  const float c1 = 1.f - std::pow(b1, (float)m->adam_t);
-  const float c2 = 1.f - std::pow(b2, (float)m->adam_t);
-  hipLaunchKernelGGL(adam_kernel, dim3(256), dim3(256), 0, m->stream, m->n_params, m->d_p,
-                     m->d_g, m->d_m, m->d_v, lr, b1, b2, 1e-8f, c1, c2);
+  hipLaunchKernelGGL(adam_kernel, dim3(256), dim3(256), 0, m->stream, m->n_params, m->d_g,
+                     adam_args(m, lr));
   MLPCHK(hipGetLastError());
+  if (int rc = pack(m)) return rc;
   MLPCHK(hipStreamSynchronize(m->stream));
   return SCFT_OK;
 }
@@ -515,7 +1031,6 @@ extern "C" int scft_mlp_train(scft_mlp* m, int n_samples, const float* X, const 
   std::vector<int> idx(n_samples);
   for (int i = 0; i < n_samples; i++) idx[i] = i;
   uint64_t s = seed;
-  const float b1 = 0.9f, b2 = 0.999f;
   if (hipMemcpy(dX, xn.data(), sizeof(float) * xn.size(), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(dY, yn.data(), sizeof(float) * yn.size(), hipMemcpyHostToDevice) != hipSuccess)
     rc = SCFT_E_HIP;
@@ -537,6 +1052,12 @@ extern "C" int scft_mlp_train(scft_mlp* m, int n_samples, const float* X, const 
     }
     for (int b0 = 0; b0 < n_samples && rc == SCFT_OK; b0 += batch) {
       const int nb = std::min(batch, n_samples - b0);
+      if (m->whole) {  // two launches: rows, then weights
+        m->adam_t++;
+        const AdamArgs adam = adam_args(m, lr);
+        if (run_net(m, nb, dX, dY, dIdx + b0) || run_grad(m, nb, &adam)) rc = SCFT_E_HIP;
+        continue;
+      }
       hipLaunchKernelGGL(gather_kernel, dim3(128), dim3(256), 0, m->stream, dX, dIdx + b0, nb,
                          din, m->d_act[0]);
       hipLaunchKernelGGL(gather_kernel, dim3(128), dim3(256), 0, m->stream, dY, dIdx + b0, nb,
@@ -546,10 +1067,8 @@ extern "C" int scft_mlp_train(scft_mlp* m, int n_samples, const float* X, const 
         break;
       }
       m->adam_t++;
-      const float c1 = 1.f - std::pow(b1, (float)m->adam_t);
-      const float c2 = 1.f - std::pow(b2, (float)m->adam_t);
-      hipLaunchKernelGGL(adam_kernel, dim3(256), dim3(256), 0, m->stream, m->n_params, m->d_p,
-                         m->d_g, m->d_m, m->d_v, lr, b1, b2, 1e-8f, c1, c2);
+      hipLaunchKernelGGL(adam_kernel, dim3(256), dim3(256), 0, m->stream, m->n_params, m->d_g,
+                         adam_args(m, lr));
       if (hipGetLastError() != hipSuccess) rc = SCFT_E_HIP;
     }
     // also orders the next epoch's host shuffle after this epoch's index copy
