@@ -111,9 +111,13 @@ inline int bucket_capacity(int n) {
 // Euler: one wave up to 512 unknowns, then waves of 8 rows per lane; the 1024
 // bucket takes 4 waves of 4 rows while every instance finds a CU of its own
 // (a step 0.37 us against 0.47 us at <8, 2>), and <8, 2> beyond (1030 against
-// 860 G node-steps/s with the chip full).  IRK4 keeps ~11 doubles per row.
+// 860 G node-steps/s with the chip full).  IRK4 keeps ~11 doubles per row and
+// is bound by a wave's own instructions, so there the 512 bucket does likewise
+// (600-1000 unknowns, <= 256 instances, 512 steps: <4, 4> 0.50-0.58 ms against
+// <8, 2> 0.65-0.69; 300 unknowns <4, 2> 0.40-0.43 against <8, 1> 0.41-0.47; with
+// 1024 instances 0.93 against 0.61).
 inline int bucket_default_K(int cap, bool irk4, int items, int cus) {
-  if (!irk4 && cap == 1024 && items <= cus) return 4;
+  if ((cap == 1024 || (irk4 && cap == 512)) && items <= cus) return 4;
   const int k = cap / 64;
   return k < 8 ? k : 8;
 }

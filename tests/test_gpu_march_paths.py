@@ -80,3 +80,21 @@ def test_small_sizes_in_one_launch():
 def test_pairing_weights_by_class(N):
     import scft_amd as S
     _check(S, [_make(40, N, 3.0, O.BC_DD, 5)], O.BC_DD)
+
+
+@pytest.mark.parametrize("n", [257, 511, 512, 513, 1000, 1024])
+def test_irk4_rows_per_lane(n):
+    """IRK4 buckets of 512 and 1024 unknowns take four rows per lane while every
+    instance finds a CU, eight beyond."""
+    import scft_amd as S
+    bc, cmat, N = O.BC_DN, O.C_CONSISTENT, 32
+    it = _make(n, N, 4.0, bc, n)
+    ref = O.evaluate(it["x"], it["w"], it["pt"], N, bc=bc, cmat=cmat, stepper=O.STEP_IRK4)
+    for count in (1, 700):
+        b = S.Batch([it["x"]] * count, [N] * count, [unknowns(it["pt"], bc)] * count, bc=bc, cmat=cmat,
+                    stepper=S.STEP_IRK4)
+        out = b.eval([unknowns(it["w"], bc)] * count)
+        b.close()
+        assert (out["status"] == 0).all()
+        for phi in out["phi"]:
+            np.testing.assert_allclose(phi, unknowns(ref["phi"], bc), rtol=0, atol=PHI_ATOL)
