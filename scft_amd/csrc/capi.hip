@@ -908,9 +908,15 @@ extern "C" int scft_batch_autotune(scft_batch* b, int reps) {
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
   const int nb = static_cast<int>(b->buckets.size());
+  bool together = false;
+  for (auto& l : b->launches) together = together || l.small;
   for (int bi = 0; bi < nb; bi++) {
     Bucket& bk = b->buckets[bi];
     if (bk.items.empty() || bk.dense) continue;  // (the dense march has one variant)
+    // Buckets that share a launch stay in it: a variant or grid that suits one
+    // of them alone would give each its own launch again (4096 uniform meshes,
+    // a sweep 10.0 ms together, 10.8 with seven launches each at its best).
+    if (together && bk.cap <= 512) continue;
     float best = 1e30f;
     int bestK = bk.K, bestW = bk.W, bestP = bk.wpc;
     for (int K : Ks)
