@@ -34,8 +34,11 @@ Also reported:
                 of its converged field against the CPU oracle's evaluation of
                 the same field, and the oracle's residual of it
   roofline      the dominant march launch (largest per-bucket time) of one
-                evaluation sweep: algorithmic bytes (q-slabs written and read
-                back, O(n) I/O) over its HIP-event duration, against 8 TB/s
+                evaluation sweep: algorithmic bytes (the q-slabs it keeps, written
+                and read back, O(n) I/O) over its HIP-event duration, against
+                8 TB/s.  A batch that fills the chip keeps every fourth slab
+                and recomputes the others, so that HBM no longer bounds it but
+                the FP64 vector units do
   cpu_baseline  the CPU oracle (same mixer, same tolerance, cold start) on a
                 bounded sample of the same instances, threads over the host
                 cores the GPU box allots to one GPU; beside it the reference
@@ -187,7 +190,7 @@ def march_source_sha256():
     it inlines: slab layout and access, lane moves)."""
     import hashlib
     h = hashlib.sha256()
-    for name in ("march.hip", "device_common.h"):
+    for name in ("march.hip", "march_rows.h", "device_common.h"):
         with open(os.path.join(ROOT, "scft_amd", "csrc", name), "rb") as f:
             h.update(f.read())
     return h.hexdigest()

@@ -221,11 +221,12 @@ typedef struct scft_anderson_opts {
                              evaluations than the linear form throughout.
                              0: the rational form from the first update */
   int inner_sweeps;       /* k >= 1 (0 counts as 1): within each sweep after
-                             the first, the instances of the size buckets
+                             the first, the instances of the launches
+                             (a size bucket, or the small ones together)
                              with at most a third of the work of the
                              largest go through k evaluations and mixer
-                             updates, on their own streams while the
-                             largest marches once.  Every instance takes
+                             updates, beside the largest, which marches
+                             once.  Every instance takes
                              the same evaluations and updates in the same
                              order as with 1 (the results are the same
                              bits); the solve needs fewer sweeps when small
@@ -241,7 +242,8 @@ typedef struct scft_solve_stats {
   double seconds;         /* wall time of the solve (device resident) */
   double eval_seconds;    /* part spent in the march kernels (events) */
   double node_steps;      /* sum over evaluations of n * N */
-  double bytes;           /* sum over evaluations of the algorithmic bytes */
+  double bytes;           /* sum over evaluations of the algorithmic bytes
+                             of a march that keeps every slab */
 } scft_solve_stats;
 
 /* w: in = initial fields, out = solutions (host, on unknowns); w_cold

@@ -12,8 +12,8 @@
 // omega = 1 - i sqrt3 (the product of the first entries of 1^T V and
 // V^{-1} 1 for Ah's eigenvector matrix V; on a scalar problem q' = -mu q this
 // reproduces the Gauss method's factor (1 - y/2 + y^2/12) / (1 + y/2 + y^2/12),
-// y = mu dt).  So a step is one complex tridiagonal solve, with the
-// implicit-Euler march's structure (march.hip) carried over complex numbers:
+// y = mu dt).  So a step is one complex tridiagonal solve, by elimination down
+// and substitution up:
 //
 //   setup   rows of A and D' from the mesh and the field, S = A + dt lambda D'
 //           (complex), Thomas pivots of S from a wave/workgroup prefix product
@@ -27,12 +27,16 @@
 //           (broadcast DPP forward, LDS-crossbar permutes backward) and a
 //           fold over waves through LDS, with every multiplier fixed per
 //           instance;
-//   density and residual exactly as march.hip: slabs 1 .. N/2-1 streamed to
+//   density and residual: slabs 1 .. N/2-1 streamed to
 //           HBM and paired with steps N/2+1 .. N through a register ring,
 //           Romberg pairing weights in LDS, r = phi - phi_t, ||r||_inf.
 //
 // Per step and row this is 14 flops against implicit Euler's ~6, and twice
-// the lane moves; the HBM traffic per evaluation is the same.
+// the lane moves; the HBM traffic per evaluation is the same.  Bound by a wave's
+// own instructions (~30 FP64 per row and step): march.hip's form, two
+// recurrences side by side with one exchange, gains nothing here (100-300
+// unknowns within 5%) and its second set of multipliers spills at 8 rows per
+// lane and several waves (600 unknowns 1.29 ms for 512 steps against 0.65).
 #include "scft_internal.h"
 #include "device_common.h"
 #include "march_rows.h"
