@@ -65,6 +65,7 @@ struct Bucket {
   std::vector<int> items;  // instance ids, largest cost first
   int* d_items = nullptr;
   int grid = 0;
+  int seg = 1;    // slabs kept: every one, or every seg-th (march.hip)
   int dense = 0;  // width of the dense march (dense.hip), 0: the scan march
   int wpc = 0;  // workgroups per CU of the persistent grid (0: as many as fit)
   long long slab_stride = 0;  // doubles per workgroup
@@ -102,7 +103,6 @@ struct scft_batch {
   std::vector<Bucket> buckets;
   std::vector<Launch> launches;  // of one sweep, longest expected run first
   int* d_small_items = nullptr;  // the items of a small launch
-  int seg = 1;                   // slabs kept: every one, or every seg-th (march.hip)
   hipStream_t stream = nullptr;  // main stream: copies, resets, the mixer
   // Buckets run concurrently on the main stream plus kSide side streams.  A
   // process has four hardware queues: more streams share them, and a shared
@@ -248,10 +248,18 @@ static int size_scratch(scft_batch* b) {
   // every MARCH_SEG-th and march 1.375 times as many steps.  Sweeps measured
   // both ways, all slabs / every fourth: 1024 uniform meshes (0.8 of the
   // longest chain) 4.5 / 5.1 ms, 1024 graded (1.2) 9.5 / 11.2; 4096 uniform
-  // (2.9) 12.1 / 10.5, 4096 graded (3.0) 28.5 / 25.8.  A single instance
-  // keeps all of them (scft_debug_slabs reads them).
+  // (2.9) 12.1 / 10.5, 4096 graded (3.0) 28.5 / 25.8.  In between, launches that
+  // end well before the longest chain even with the extra steps keep every
+  // MARCH_SEG-th, which leaves more of HBM to the others: 1024 uniform 4.07 ->
+  // 3.87 ms, 1024 graded 8.28 -> 7.91 (2048: no difference).  A single
+  // instance keeps all of them (scft_debug_slabs reads them).
   const double traffic_us = b->bytes_all / 5.0e6;
-  b->seg = (!irk4 && b->n_inst > 1 && traffic_us > 1.6 * longest) ? MARCH_SEG : 1;
+  const bool may = !irk4 && b->n_inst > 1;
+  const bool all_seg = may && traffic_us > 1.6 * longest;
+  const bool some_seg = may && traffic_us > 0.5 * longest;
+  auto seg_for = [&](double us) {  // `us`: the expected run with every slab kept
+    return all_seg || (some_seg && 1.375 * us < 0.9 * longest) ? MARCH_SEG : 1;
+  };
 
   b->launches.clear();
   long long need = 0;
@@ -259,16 +267,29 @@ static int size_scratch(scft_batch* b) {
   // one launch for the small buckets when there are more launches than
   // hardware queues (march_small_kernel)
   const bool merge = small_ok && small >= 2 && filled > 1 + scft_batch::kSide;
+  int group_seg = 1;
   std::vector<std::pair<double, int>> merged;
   long long group_need = 0;
+  if (merge) {
+    double us = 0.0, most = 0.0;
+    for (auto& bk : b->buckets)
+      for (int k : bk.items)
+        if (bk.cap <= 512) {
+          const double t = step_us(bk.K, bk.W) * b->desc[k].N;
+          us += t;
+          most = std::max(most, t);
+        }
+    group_seg = seg_for(std::max(most, us / std::max(1, march_small_max_grid(MARCH_SEG))));
+  }
   for (size_t i = 0; i < b->buckets.size(); i++) {
     Bucket& bk = b->buckets[i];
     if (bk.items.empty()) continue;
     const bool in_group = merge && bk.cap <= 512;
-    bk.grid = std::max(1, grid_of(bk, b->seg));
-    const long long kept = std::max(1, bk.Nmax / 2 / b->seg);
+    bk.seg = bk.dense ? 1 : in_group ? group_seg : seg_for(run_us(b, bk, grid_of(bk, MARCH_SEG)));
+    bk.grid = std::max(1, grid_of(bk, bk.seg));
+    const long long kept = std::max(1, bk.Nmax / 2 / bk.seg);
     bk.slab_stride = bk.dense ? static_cast<long long>(bk.Nmax / 2) * bk.dense
-                              : kept * march_slab_len(bk.K, bk.W, b->seg);
+                              : kept * march_slab_len(bk.K, bk.W, bk.seg);
     bk.slab_base = need;
     double work = 0.0;
     for (int k : bk.items) work += static_cast<double>(b->desc[k].n) * b->desc[k].N;
@@ -311,9 +332,9 @@ static int size_scratch(scft_batch* b) {
                      hipMemcpyHostToDevice));
     group.d_items = b->d_small_items;
     group.n_items = static_cast<int>(ids.size());
-    group.grid = std::max(1, std::min(group.n_items, march_small_max_grid(b->seg)));
-    group.slab_stride = std::max<long long>(1, group.Nmax / 2 / b->seg) *
-                        march_slab_len(8, 1, b->seg);
+    group.grid = std::max(1, std::min(group.n_items, march_small_max_grid(group_seg)));
+    group.slab_stride = std::max<long long>(1, group.Nmax / 2 / group_seg) *
+                        march_slab_len(8, 1, group_seg);
     // the small buckets are the first ones: their region starts the scratch
     group.slab_base = 0;
     group_need = std::max(group_need, group.slab_stride * group.grid);
@@ -387,7 +408,7 @@ static MarchArgs march_args(const scft_batch* b, const Bucket& bk, int bucket_id
   a.slabs = b->d_slabs + bk.slab_base;
   a.slab_stride = bk.slab_stride;
   a.half_max = bk.Nmax / 2;
-  a.seg = b->seg;
+  a.seg = bk.seg;
   a.items = bk.d_items;
   a.queue = b->d_counters + bucket_idx;
   a.n_items = static_cast<int>(bk.items.size());
@@ -815,7 +836,7 @@ extern "C" int scft_batch_time_buckets(scft_batch* b, const double* w, int reps,
     if (c < max_buckets) {
       if (ms) ms[c] = t / reps;
       double by = 0.0;
-      for (int k : bk.items) by += slab_bytes(b->desc[k].n, b->desc[k].N, b->seg);
+      for (int k : bk.items) by += slab_bytes(b->desc[k].n, b->desc[k].N, bk.seg);
       if (bytes) bytes[c] = by;
       if (n_items) n_items[c] = static_cast<int>(bk.items.size());
     }
@@ -923,7 +944,7 @@ extern "C" int scft_batch_autotune(scft_batch* b, int reps) {
       for (int W : Wsz) {
         if (64 * K * W < bk.nmax || 64 * K * W > 2 * bk.cap) continue;
         if (!variant_exists(b, K, W)) continue;
-        const int mg = eval_max_grid(b, K, W, bk.Nmax / 2, b->seg);
+        const int mg = eval_max_grid(b, K, W, bk.Nmax / 2, bk.seg);
         if (mg < 1) continue;
         const int occ = std::max(1, mg / b->cus);
         for (int wpc = 1; wpc <= occ; wpc++) {
