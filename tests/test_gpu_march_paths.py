@@ -76,6 +76,28 @@ def test_small_sizes_in_one_launch():
     _check(S, few + [big] * 700, O.BC_DN)
 
 
+@pytest.mark.parametrize("ns", [[100, 500], [40, 100, 200, 500, 1000]], ids=["buckets", "grouped"])
+def test_some_launches_recompute(ns):
+    """Slab traffic between the two regimes: the launches of small instances
+    keep every fourth slab, the one large instance, the longest chain, all."""
+    import scft_amd as S
+    bc = O.BC_DN
+    base = [_make(n, 64, 3.0, bc, n) for n in ns]
+    big = _make(4095, 128, 6.0, bc, 7)
+    mean = sum(ns) / len(ns)
+    count = int(0.7 * 80.0 * 5.0e6 / (8.0 * mean * 64)) // len(ns)  # 0.7 of ~80 us at 5 TB/s
+    insts = base * count + [big]
+    _check(S, insts, bc)
+    b = S.Batch([it["x"] for it in insts], [it["N"] for it in insts],
+                [unknowns(it["pt"], bc) for it in insts], bc=bc)
+    times = b.time_buckets(b.join([unknowns(it["w"], bc) for it in insts]), 1)
+    b.close()
+    for (items, _, nbytes), it in zip(times, base + [big]):
+        n, N = len(it["x"]) - 1, it["N"]
+        kept = 8.0 * n * (N - 2) if it is big else 8.0 * n * 2 * (N // 8)
+        assert nbytes == items * (kept + 40.0 * n)
+
+
 @pytest.mark.parametrize("N", [16, 32, 64, 128])
 def test_pairing_weights_by_class(N):
     import scft_amd as S
