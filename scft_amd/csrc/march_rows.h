@@ -183,9 +183,11 @@ __device__ __forceinline__ void inverse_rows(const double (&av)[K], const double
     A = An;
     Dd = Bd;
     Bd = Bn;
-    if (t % 4 == 3 && t + 1 < K) norm4(A, Cd, Bd, Dd);
+    // every second row (the last is one): the product of four rows overflows at
+    // 1e77, of two where a row's own products do
+    if (t % 2 == 1) norm4(A, Cd, Bd, Dd);
   }
-  norm4(A, Cd, Bd, Dd);
+  if constexpr (K == 1) norm4(A, Cd, Bd, Dd);
   // Adjacent chunks combine as a 2x2 product, whichever side's matrix carries
   // the coupling: the prefix form T = [[A, C], [-p_left B, -p_left D]] gives
   // the pivot of the last row before a chunk, T00 / T01; the suffix form
