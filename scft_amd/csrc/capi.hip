@@ -89,6 +89,7 @@ struct Launch {
 }  // namespace
 
 constexpr size_t kStageBytes = size_t(256) << 10;
+constexpr long long kMergeDoubles = (4ll << 30) / 8;
 
 struct scft_batch {
   int device = 0;
@@ -264,9 +265,18 @@ static int size_scratch(scft_batch* b) {
   b->launches.clear();
   long long need = 0;
   Launch group;
+  // how a bucket is launched by itself
+  auto shape = [&](Bucket& bk, int seg) {
+    bk.seg = seg;
+    bk.grid = std::max(1, grid_of(bk, seg));
+    const long long kept = std::max(1, bk.Nmax / 2 / seg);
+    bk.slab_stride = bk.dense ? static_cast<long long>(bk.Nmax / 2) * bk.dense
+                              : kept * march_slab_len(bk.K, bk.W, seg);
+    return bk.slab_stride * bk.grid;
+  };
   // one launch for the small buckets when there are more launches than
   // hardware queues (march_small_kernel)
-  const bool merge = small_ok && small >= 2 && filled > 1 + scft_batch::kSide;
+  bool merge = small_ok && small >= 2 && filled > 1 + scft_batch::kSide;
   int group_seg = 1;
   std::vector<std::pair<double, int>> merged;
   long long group_need = 0;
@@ -278,18 +288,37 @@ static int size_scratch(scft_batch* b) {
           const double t = step_us(bk.K, bk.W) * b->desc[k].N;
           us += t;
           most = std::max(most, t);
+          group.n_items++;
         }
     group_seg = seg_for(std::max(most, us / std::max(1, march_small_max_grid(MARCH_SEG))));
+    group.grid = std::max(1, std::min(group.n_items, march_small_max_grid(group_seg)));
+    // Any workgroup may take any of them, so a region holds the largest.  One by
+    // one the launches may need far less (thousands of the smallest sizes
+    // beside a few of 512 unknowns: 2 GB against 17), so they stay apart where
+    // the scratch would grow by more than a quarter and 4 GiB: mixes of 32 to
+    // 16384 instances need 0.82 to 1.15 of it.  Together / apart, sweeps in us:
+    // 4096 of 31 unknowns and one each of four larger sizes, 512 steps, 352 /
+    // 406; 2048 of 59 and five, 1024 steps, 630 / 790.
+    long long apart = 0, rest = 0;
+    for (auto& bk : b->buckets) {
+      if (bk.items.empty()) continue;
+      const long long own = shape(bk, seg_for(run_us(b, bk, grid_of(bk, MARCH_SEG))));
+      (bk.cap <= 512 ? apart : rest) += own;
+      if (bk.cap <= 512) {
+        group_need = std::max(group_need, shape(bk, group_seg));
+        group.slab_stride = std::max(group.slab_stride, bk.slab_stride);
+      }
+    }
+    group_need = std::max(group_need, group.slab_stride * group.grid);
+    merge = group_need + rest <= apart + rest + std::max((apart + rest) / 4, kMergeDoubles);
+    if (!merge) group_need = 0;
   }
   for (size_t i = 0; i < b->buckets.size(); i++) {
     Bucket& bk = b->buckets[i];
     if (bk.items.empty()) continue;
     const bool in_group = merge && bk.cap <= 512;
-    bk.seg = bk.dense ? 1 : in_group ? group_seg : seg_for(run_us(b, bk, grid_of(bk, MARCH_SEG)));
-    bk.grid = std::max(1, grid_of(bk, bk.seg));
-    const long long kept = std::max(1, bk.Nmax / 2 / bk.seg);
-    bk.slab_stride = bk.dense ? static_cast<long long>(bk.Nmax / 2) * bk.dense
-                              : kept * march_slab_len(bk.K, bk.W, bk.seg);
+    const long long own = shape(bk, bk.dense ? 1 : in_group ? group_seg
+                                        : seg_for(run_us(b, bk, grid_of(bk, MARCH_SEG))));
     bk.slab_base = need;
     double work = 0.0;
     for (int k : bk.items) work += static_cast<double>(b->desc[k].n) * b->desc[k].N;
@@ -299,11 +328,10 @@ static int size_scratch(scft_batch* b) {
       group.small = true;
       group.Nmax = std::max(group.Nmax, bk.Nmax);
       group.work += work;
-      group_need = std::max(group_need, bk.slab_stride * bk.grid);
       for (int k : bk.items) merged.push_back({step_us(bk.K, bk.W) * b->desc[k].N, k});
       continue;
     }
-    need += bk.slab_stride * bk.grid;
+    need += own;
     Launch l;
     l.bucket = static_cast<int>(i);
     l.d_items = bk.d_items;
@@ -331,13 +359,8 @@ static int size_scratch(scft_batch* b) {
     HIPCHK(hipMemcpy(b->d_small_items, ids.data(), sizeof(int) * ids.size(),
                      hipMemcpyHostToDevice));
     group.d_items = b->d_small_items;
-    group.n_items = static_cast<int>(ids.size());
-    group.grid = std::max(1, std::min(group.n_items, march_small_max_grid(group_seg)));
-    group.slab_stride = std::max<long long>(1, group.Nmax / 2 / group_seg) *
-                        march_slab_len(8, 1, group_seg);
     // the small buckets are the first ones: their region starts the scratch
     group.slab_base = 0;
-    group_need = std::max(group_need, group.slab_stride * group.grid);
     for (auto& l : b->launches) l.slab_base += group_need;
     for (auto& bk : b->buckets)
       if (bk.cap > 512) bk.slab_base += group_need;
