@@ -193,13 +193,20 @@ static double step_us(int K, int W) {
 
 // A persistent grid's expected run: its longest instance, or all of them
 // spread over the workgroups.
-static double run_us(const scft_batch* b, const Bucket& bk, int grid) {
+static double run_us(const scft_batch* b, const Bucket& bk, int K, int W, int grid) {
   if (bk.dense)  // ~35 / 110 us to build the powers, then 64 steps at a time
     return (bk.dense == 32 ? 35.0 + 0.008 * bk.Nmax : 110.0 + 0.03 * bk.Nmax) *
            ((bk.items.size() + grid - 1) / std::max(1, grid));
   double steps = 0.0;
   for (int k : bk.items) steps += b->desc[k].N;
-  return step_us(bk.K, bk.W) * std::max<double>(bk.Nmax, steps / std::max(1, grid));
+  return step_us(K, W) * std::max<double>(bk.Nmax, steps / std::max(1, grid));
+}
+
+// Rows per lane and waves of a bucket before any tuning.
+static void untuned(const scft_batch* b, const Bucket& bk, int* K, int* W) {
+  *K = bucket_default_K(bk.cap, b->stepper == SCFT_STEP_IRK4, static_cast<int>(bk.items.size()),
+                        b->cus);
+  *W = bk.cap / 64 / *K;
 }
 
 // Every launch of a sweep owns a scratch region (they run concurrently): grid
@@ -215,6 +222,17 @@ static int size_scratch(scft_batch* b) {
     // longest instances set the makespan, and they step faster alone
     const int cap_grid = bk.wpc > 0 ? std::min(mg, bk.wpc * b->cus) : mg;
     return std::min<int>(static_cast<int>(bk.items.size()), cap_grid);
+  };
+  // The expected run of a bucket before any tuning.  It decides which slabs are
+  // kept: from the tuned grid, a candidate of the autotuner with few workgroups
+  // would be the longest chain, put the batch on every slab, and be timed
+  // against candidates that keep every fourth.
+  auto untuned_us = [&](const Bucket& bk, int seg) {
+    int K, W;
+    untuned(b, bk, &K, &W);
+    const int mg = bk.dense ? dense_max_grid(bk.dense, irk4)
+                            : eval_max_grid(b, K, W, bk.Nmax / 2, seg);
+    return run_us(b, bk, K, W, std::min<int>(static_cast<int>(bk.items.size()), mg));
   };
   int filled = 0, small = 0;
   for (auto& bk : b->buckets) filled += bk.items.empty() ? 0 : 1;
@@ -232,8 +250,7 @@ static int size_scratch(scft_batch* b) {
       for (int k : bk.items) Nmin = std::min(Nmin, b->desc[k].N);
       bk.dense = dense_width(bk.nmax, Nmin, static_cast<int>(bk.items.size()), b->cus, irk4);
     }
-    const int g = grid_of(bk, 1);
-    if (g < 1) {
+    if (grid_of(bk, 1) < 1) {
       snprintf(g_errmsg, sizeof g_errmsg, "march variant K=%d W=%d does not fit a CU", bk.K,
                bk.W);
       return SCFT_E_ARG;
@@ -242,7 +259,7 @@ static int size_scratch(scft_batch* b) {
       small++;
       small_ok = small_ok && bk.W == 1 && bk.K == bk.cap / 64 && bk.wpc == 0;
     }
-    longest = std::max(longest, run_us(b, bk, g));
+    longest = std::max(longest, untuned_us(bk, 1));
   }
   // Keep every slab while their traffic (at the ~5 TB/s that mixed stores and
   // loads reach) takes less time than the longest chain of steps; else keep
@@ -302,7 +319,7 @@ static int size_scratch(scft_batch* b) {
     long long apart = 0, rest = 0;
     for (auto& bk : b->buckets) {
       if (bk.items.empty()) continue;
-      const long long own = shape(bk, seg_for(run_us(b, bk, grid_of(bk, MARCH_SEG))));
+      const long long own = shape(bk, seg_for(untuned_us(bk, MARCH_SEG)));
       (bk.cap <= 512 ? apart : rest) += own;
       if (bk.cap <= 512) {
         group_need = std::max(group_need, shape(bk, group_seg));
@@ -318,7 +335,7 @@ static int size_scratch(scft_batch* b) {
     if (bk.items.empty()) continue;
     const bool in_group = merge && bk.cap <= 512;
     const long long own = shape(bk, bk.dense ? 1 : in_group ? group_seg
-                                        : seg_for(run_us(b, bk, grid_of(bk, MARCH_SEG))));
+                                        : seg_for(untuned_us(bk, MARCH_SEG)));
     bk.slab_base = need;
     double work = 0.0;
     for (int k : bk.items) work += static_cast<double>(b->desc[k].n) * b->desc[k].N;
@@ -341,7 +358,7 @@ static int size_scratch(scft_batch* b) {
     l.slab_stride = bk.slab_stride;
     l.slab_base = bk.slab_base;
     l.work = work;
-    l.us = run_us(b, bk, bk.grid);
+    l.us = run_us(b, bk, bk.K, bk.W, bk.grid);
     b->launches.push_back(l);
   }
   if (merge) {
@@ -630,11 +647,7 @@ extern "C" int scft_batch_create(scft_batch** out, const scft_batch_desc* dsc) {
         bk.Nmax = std::max(bk.Nmax, b->desc[k].N);
       }
   }
-  for (auto& bk : b->buckets) {
-    bk.K = bucket_default_K(bk.cap, b->stepper == SCFT_STEP_IRK4,
-                            static_cast<int>(bk.items.size()), b->cus);
-    bk.W = bk.cap / 64 / bk.K;
-  }
+  for (auto& bk : b->buckets) untuned(b, bk, &bk.K, &bk.W);
   read_tune_file(b);
 
   int rc = SCFT_OK;
@@ -967,12 +980,15 @@ extern "C" int scft_batch_autotune(scft_batch* b, int reps) {
       for (int W : Wsz) {
         if (64 * K * W < bk.nmax || 64 * K * W > 2 * bk.cap) continue;
         if (!variant_exists(b, K, W)) continue;
+        if (eval_max_grid(b, K, W, bk.Nmax / 2, 1) < 1) continue;
+        bk.K = K;
+        bk.W = W;
+        bk.wpc = 0;
+        SCFT_TRY(size_scratch(b));  // (the slabs it keeps, which its occupancy depends on)
         const int mg = eval_max_grid(b, K, W, bk.Nmax / 2, bk.seg);
         if (mg < 1) continue;
         const int occ = std::max(1, mg / b->cus);
         for (int wpc = 1; wpc <= occ; wpc++) {
-          bk.K = K;
-          bk.W = W;
           bk.wpc = (wpc == occ) ? 0 : wpc;
           SCFT_TRY(size_scratch(b));
           MarchArgs a = march_args(b, bk, bi);

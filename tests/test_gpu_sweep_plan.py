@@ -49,3 +49,22 @@ def test_scratch_of_many_small_instances_beside_a_few_larger():
         for j in (k, k + c - 1):
             np.testing.assert_allclose(out["phi"][j], unknowns(ref["phi"], BC), rtol=0, atol=1e-10)
         k += c
+
+
+def test_tuning_does_not_change_which_slabs_are_kept():
+    """One workgroup per CU (as a candidate of the autotuner, or from a tune file)
+    makes the launch longer, not its slab traffic: the slabs kept follow from the
+    sizes alone, and so do the bytes that time_buckets reports."""
+    import tempfile
+
+    import scft_amd as S
+    parts = [(100, 64, 6000)]
+    kept = 6000 * (8.0 * 100 * 2 * (64 // 2 // 4) + 40.0 * 100)
+    with tempfile.NamedTemporaryFile("w", suffix=".txt") as f:
+        f.write("128 2 1 1\n")
+        f.flush()
+        for tune in (None, f.name):
+            b, w, _ = _batch(S, parts, tune_file=tune)
+            (items, _, nbytes), = b.time_buckets(w, 1)
+            b.close()
+            assert (items, nbytes) == (6000, kept), tune
