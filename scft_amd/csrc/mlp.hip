@@ -518,7 +518,7 @@ struct scft_mlp {
   std::vector<int> dims;           // dims[0] inputs ... dims[L] outputs
   std::vector<long long> off;      // parameter offset of each layer
   long long n_params = 0;
-  int cap_batch = 0;               // activation buffers sized for this batch
+  int cap_batch = 0, cap_train = 0;  // rows that the buffers of each pass hold
   float *d_p = nullptr, *d_g = nullptr, *d_m = nullptr, *d_v = nullptr;
   std::vector<float*> d_act;       // L + 1 activation buffers [cap_batch x dims[l]]
   float *d_delta0 = nullptr, *d_delta1 = nullptr, *d_t = nullptr;
@@ -551,33 +551,60 @@ int mlp_dalloc(float** p, long long n) {
              : SCFT_E_NOMEM;
 }
 
-void free_batch(scft_mlp* m) {
-  for (auto p : m->d_act) (void)hipFree(p);
+// Row buffers of a forward pass (the hidden activations of a whole network stay
+// in LDS), and what training needs beside them.  A forward pass of many rows
+// then does not pay for deltas: 200 000 rows of 133 - 4 x 256 - 136 take 0.2 GB,
+// 2.1 GB with everything.
+void free_forward(scft_mlp* m) {
+  for (size_t l = 0; l < m->d_act.size(); l++) {
+    if (m->whole && l > 0 && l + 1 < m->d_act.size()) continue;
+    (void)hipFree(m->d_act[l]);
+    m->d_act[l] = nullptr;
+  }
+  m->cap_batch = 0;
+}
+
+void free_train(scft_mlp* m) {
+  for (size_t l = 1; m->whole && l + 1 < m->d_act.size(); l++) {
+    (void)hipFree(m->d_act[l]);
+    m->d_act[l] = nullptr;
+  }
   for (auto p : m->d_delta) (void)hipFree(p);
   (void)hipFree(m->d_delta0);
   (void)hipFree(m->d_delta1);
   (void)hipFree(m->d_t);
-  m->d_act.assign(m->dims.size(), nullptr);
   m->d_delta.assign(m->dims.size() - 1, nullptr);
   m->d_delta0 = m->d_delta1 = m->d_t = nullptr;
-  m->cap_batch = 0;
+  m->cap_train = 0;
 }
 
-int ensure_batch(scft_mlp* m, int batch) {
-  if (batch <= m->cap_batch) return SCFT_OK;
-  free_batch(m);
-  int widest = 0;
-  for (size_t l = 0; l < m->dims.size(); l++) {
-    if (mlp_dalloc(&m->d_act[l], (long long)batch * m->dims[l])) return SCFT_E_NOMEM;
-    widest = std::max(widest, m->dims[l]);
-    if (m->whole && l > 0 && mlp_dalloc(&m->d_delta[l - 1], (long long)batch * m->dims[l]))
-      return SCFT_E_NOMEM;
+int ensure_batch(scft_mlp* m, int batch, bool train) {
+  const size_t L = m->dims.size() - 1;
+  m->d_act.resize(L + 1, nullptr);
+  if (batch > m->cap_batch) {
+    free_forward(m);
+    for (size_t l = 0; l <= L; l++)
+      if ((!m->whole || l == 0 || l == L) &&
+          mlp_dalloc(&m->d_act[l], (long long)batch * m->dims[l]))
+        return SCFT_E_NOMEM;
+    m->cap_batch = batch;
   }
-  if (!m->whole && (mlp_dalloc(&m->d_delta0, (long long)batch * widest) ||
-                    mlp_dalloc(&m->d_delta1, (long long)batch * widest)))
-    return SCFT_E_NOMEM;
-  if (mlp_dalloc(&m->d_t, (long long)batch * m->dims.back())) return SCFT_E_NOMEM;
-  m->cap_batch = batch;
+  if (train && batch > m->cap_train) {
+    free_train(m);
+    int widest = 0;
+    for (size_t l = 0; l <= L; l++) {
+      widest = std::max(widest, m->dims[l]);
+      if (m->whole && l > 0 && l < L && mlp_dalloc(&m->d_act[l], (long long)batch * m->dims[l]))
+        return SCFT_E_NOMEM;
+      if (m->whole && l > 0 && mlp_dalloc(&m->d_delta[l - 1], (long long)batch * m->dims[l]))
+        return SCFT_E_NOMEM;
+    }
+    if (!m->whole && (mlp_dalloc(&m->d_delta0, (long long)batch * widest) ||
+                      mlp_dalloc(&m->d_delta1, (long long)batch * widest)))
+      return SCFT_E_NOMEM;
+    if (mlp_dalloc(&m->d_t, (long long)batch * m->dims.back())) return SCFT_E_NOMEM;
+    m->cap_train = batch;
+  }
   return SCFT_OK;
 }
 
@@ -850,7 +877,8 @@ extern "C" int scft_mlp_create(scft_mlp** out, int n_layers, const int* dims,
 extern "C" int scft_mlp_destroy(scft_mlp* m) {
   if (!m) return SCFT_OK;
   (void)hipStreamSynchronize(m->stream);
-  free_batch(m);
+  free_forward(m);
+  free_train(m);
   (void)hipFree(m->d_pack);
   (void)hipFree(m->d_p);
   (void)hipFree(m->d_g);
@@ -911,7 +939,7 @@ extern "C" int scft_mlp_set_normalisation(scft_mlp* m, const float* x_mean, cons
 
 extern "C" int scft_mlp_forward(scft_mlp* m, int batch, const float* X, float* Y) {
   if (!m || batch < 1 || !X || !Y) return SCFT_E_ARG;
-  if (int rc = ensure_batch(m, batch)) return rc;
+  if (int rc = ensure_batch(m, batch, false)) return rc;
   std::vector<float> xn;
   normalise_rows(m, X, batch, xn);
   MLPCHK(hipMemcpyAsync(m->d_act[0], xn.data(), sizeof(float) * xn.size(),
@@ -933,7 +961,7 @@ extern "C" int scft_mlp_forward(scft_mlp* m, int batch, const float* X, float* Y
 int scft_mlp_forward_resident(scft_mlp* m, int batch, const float* d_xn, const float** d_out,
                               const float** ym, const float** ys, int* n_out, int* n_in) {
   if (!m || batch < 1 || !d_xn || !d_out) return SCFT_E_ARG;
-  if (int rc = ensure_batch(m, batch)) return rc;
+  if (int rc = ensure_batch(m, batch, false)) return rc;
   const int din = m->dims.front();
   if (m->whole) {
     if (int rc = run_net(m, batch, d_xn, nullptr, nullptr)) return rc;
@@ -965,7 +993,7 @@ int scft_mlp_normalise_inputs(const scft_mlp* m, const float* X, int rows, float
 extern "C" int scft_mlp_loss_grad(scft_mlp* m, int batch, const float* X, const float* T,
                                   double* loss, float* grad) {
   if (!m || batch < 1 || !X || !T) return SCFT_E_ARG;
-  if (int rc = ensure_batch(m, batch)) return rc;
+  if (int rc = ensure_batch(m, batch, true)) return rc;
   const int din = m->dims.front(), dout = m->dims.back();
   MLPCHK(hipMemcpyAsync(m->d_act[0], X, sizeof(float) * (size_t)batch * din,
                         hipMemcpyHostToDevice, m->stream));
@@ -1011,7 +1039,7 @@ extern "C" int scft_mlp_train(scft_mlp* m, int n_samples, const float* X, const 
   if (!m || n_samples < 1 || !X || !Y || epochs < 1 || batch < 1 || !(lr > 0.f))
     return SCFT_E_ARG;
   const int din = m->dims.front(), dout = m->dims.back();
-  if (int rc = ensure_batch(m, batch)) return rc;
+  if (int rc = ensure_batch(m, batch, true)) return rc;
   std::vector<float> xn, yn((size_t)n_samples * dout);
   normalise_rows(m, X, n_samples, xn);
   for (int r = 0; r < n_samples; r++)

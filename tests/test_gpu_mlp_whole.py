@@ -87,3 +87,29 @@ def test_epoch_is_its_steps(dims):
     assert abs(hist[0] - losses / 50) <= 1e-6 * hist[0]
     one.close()
     all_.close()
+
+
+def test_forward_pass_of_many_rows_needs_no_training_buffers():
+    """200 000 rows: the inputs, every activation and two deltas and targets as wide
+    as the widest layer (a pass layer by layer) are 1.6 GB; a forward pass keeps its
+    inputs and outputs."""
+    import ctypes as C
+
+    import scft_amd as S
+    free, total = C.c_size_t(), C.c_size_t()
+    dims, rows = [133, 256, 256, 256, 256, 136], 200000
+    net = S.Mlp(dims, seed=3)
+    X = np.random.default_rng(1).standard_normal((rows, dims[0])).astype(np.float32)
+    assert S.lib.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    before = free.value
+    Y = net.forward(X)
+    assert S.lib.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    used = before - free.value
+    assert used < 4 * rows * (sum(dims) + 2 * 256 + 136), f"{used / 1e9:.2f} GB"
+    # training of fewer rows and passes of more and fewer after it keep to their buffers
+    net.loss_grad(X[:50], Y[:50])
+    for k in (1, 300, 7):
+        np.testing.assert_array_equal(net.forward(X[-k:]), Y[-k:])
+    loss, _ = net.loss_grad(X[:400], net.forward(X[:400]))
+    assert loss < 1e-10  # (FP32 outputs, to their roundings)
+    net.close()
