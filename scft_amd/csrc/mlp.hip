@@ -499,13 +499,34 @@ __global__ void __launch_bounds__(256) grad_kernel(GradArgs g) {
   }
 }
 
-// the packed copies of one layer's weights, after the parameters were set
-__global__ void pack_kernel(const float* __restrict__ W, int dout, int din, int jf, int jb,
-                            float* __restrict__ wf, float* __restrict__ wb) {
-  const long long n = (long long)dout * din;
-  for (long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x; k < n;
-       k += (long long)gridDim.x * blockDim.x)
-    store_packed(wf, wb, jf, jb, (int)(k / din), (int)(k % din), W[k]);
+struct PackArgs {
+  int L;
+  long long n;
+  const float *p, *g;  // (g: with ADAM)
+  AdamArgs adam;
+  struct {
+    long long off;
+    float *wf, *wb;
+    int dout, din, jf, jb;
+  } l[kMaxLayers];
+};
+
+// The packed copies of all layers' weights, after the parameters were set or,
+// with ADAM, together with the step on the gradient held: one launch (an Adam
+// step of 133 - 4 x 256 - 136 takes 15 us; with a launch per layer for the
+// copies it took 28).
+template <bool ADAM>
+__global__ void pack_kernel(PackArgs a) {
+  for (long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x; k < a.n;
+       k += (long long)gridDim.x * blockDim.x) {
+    const float v = ADAM ? adam_update(a.adam, k, a.g[k], a.p[k], a.adam.m[k], a.adam.v[k]) : a.p[k];
+    int li = 0;
+    while (li + 1 < a.L && k >= a.l[li + 1].off) li++;
+    const auto& l = a.l[li];
+    const int i = static_cast<int>(k - l.off);
+    if (i < l.dout * l.din)  // (the layer's bias follows)
+      store_packed(l.wf, l.wb, l.jf, l.jb, i / l.din, i % l.din, v);
+  }
 }
 
 }  // namespace
@@ -630,15 +651,31 @@ void plan_whole(scft_mlp* m) {
   m->lds_train = m->whole ? static_cast<int>(train) : 0;
 }
 
-int pack(scft_mlp* m) {
+// the packed copies of a whole network, with `adam` after a step
+int pack(scft_mlp* m, const AdamArgs* adam) {
   if (!m->whole) return SCFT_OK;
-  for (size_t l = 0; l + 1 < m->dims.size(); l++) {
-    const int din = m->dims[l], dout = m->dims[l + 1];
-    hipLaunchKernelGGL(pack_kernel, dim3(64), dim3(256), 0, m->stream, m->d_p + m->off[l], dout,
-                       din, ring16(din), ring16(dout), m->d_pack + m->pack_f[l],
-                       m->d_pack + m->pack_b[l]);
-    MLPCHK(hipGetLastError());
+  PackArgs a{};
+  a.L = static_cast<int>(m->dims.size()) - 1;
+  a.n = m->n_params;
+  a.p = m->d_p;
+  a.g = m->d_g;
+  if (adam) a.adam = *adam;
+  for (int l = 0; l < a.L; l++) {
+    auto& t = a.l[l];
+    t.off = m->off[l];
+    t.wf = m->d_pack + m->pack_f[l];
+    t.wb = m->d_pack + m->pack_b[l];
+    t.din = m->dims[l];
+    t.dout = m->dims[l + 1];
+    t.jf = ring16(t.din);
+    t.jb = ring16(t.dout);
   }
+  const int grid = static_cast<int>(std::min<long long>(1024, (a.n + 255) / 256));
+  if (adam)
+    hipLaunchKernelGGL(pack_kernel<true>, dim3(grid), dim3(256), 0, m->stream, a);
+  else
+    hipLaunchKernelGGL(pack_kernel<false>, dim3(grid), dim3(256), 0, m->stream, a);
+  MLPCHK(hipGetLastError());
   return SCFT_OK;
 }
 
@@ -860,7 +897,7 @@ extern "C" int scft_mlp_create(scft_mlp** out, int n_layers, const int* dims,
       hipMemset(m->d_m, 0, sizeof(float) * o) != hipSuccess ||
       hipMemset(m->d_v, 0, sizeof(float) * o) != hipSuccess ||
       (np > 0 && hipMemset(m->d_pack, 0, sizeof(float) * np) != hipSuccess) ||
-      hipStreamSynchronize(nullptr) != hipSuccess || pack(m)) {
+      hipStreamSynchronize(nullptr) != hipSuccess || pack(m, nullptr)) {
     delete m;
     return SCFT_E_HIP;
   }
@@ -905,13 +942,13 @@ extern "C" int scft_mlp_get_params(const scft_mlp* m, float* out) {
 
 extern "C" int scft_mlp_set_params(scft_mlp* m, const float* in) {
   if (!m || !in) return SCFT_E_ARG;
-  MLPCHK(hipStreamSynchronize(m->stream));
-  MLPCHK(hipMemcpy(m->d_p, in, sizeof(float) * m->n_params, hipMemcpyHostToDevice));
-  MLPCHK(hipMemset(m->d_m, 0, sizeof(float) * m->n_params));
-  MLPCHK(hipMemset(m->d_v, 0, sizeof(float) * m->n_params));
+  const size_t bytes = sizeof(float) * m->n_params;
+  MLPCHK(hipMemcpyAsync(m->d_p, in, bytes, hipMemcpyHostToDevice, m->stream));
+  MLPCHK(hipMemsetAsync(m->d_m, 0, bytes, m->stream));
+  MLPCHK(hipMemsetAsync(m->d_v, 0, bytes, m->stream));
   m->adam_t = 0;
-  MLPCHK(hipStreamSynchronize(nullptr));
-  if (int rc = pack(m)) return rc;
+  if (int rc = pack(m, nullptr)) return rc;
+  MLPCHK(hipStreamSynchronize(m->stream));
   return SCFT_OK;
 }
 
@@ -1021,10 +1058,13 @@ extern "C" int scft_mlp_loss_grad(scft_mlp* m, int batch, const float* X, const 
 extern "C" int scft_mlp_adam_step(scft_mlp* m, float lr) {
   if (!m) return SCFT_E_ARG;
   m->adam_t++;
-  hipLaunchKernelGGL(adam_kernel, dim3(256), dim3(256), 0, m->stream, m->n_params, m->d_g,
-                     adam_args(m, lr));
-  MLPCHK(hipGetLastError());
-  if (int rc = pack(m)) return rc;
+  const AdamArgs adam = adam_args(m, lr);
+  if (m->whole) {
+    if (int rc = pack(m, &adam)) return rc;
+  } else {
+    hipLaunchKernelGGL(adam_kernel, dim3(256), dim3(256), 0, m->stream, m->n_params, m->d_g, adam);
+    MLPCHK(hipGetLastError());
+  }
   MLPCHK(hipStreamSynchronize(m->stream));
   return SCFT_OK;
 }
