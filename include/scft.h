@@ -136,7 +136,12 @@ int scft_batch_destroy(scft_batch *b);
 int scft_batch_layout(const scft_batch *b, long long *uoff, long long *total);
 
 /* One field evaluation of every instance (host buffers on unknowns):
- * phi (nullable), r = phi - phi_t, rnorm[k] = ||r_k||_inf, status[k]. */
+ * phi (nullable), r = phi - phi_t, rnorm[k] = ||r_k||_inf, status[k].
+ * Evaluations of one batch repeat each other's bits.  The march that an
+ * instance goes through (rows per lane, slabs kept or recomputed, the dense
+ * form of small meshes) is chosen for the batch it is in, so the same instance
+ * alone, in a shard or in another batch agrees to rounding (1e-13 of phi), not
+ * bit for bit. */
 int scft_batch_eval(scft_batch *b, const double *w, double *phi, double *r,
                     double *rnorm, unsigned *status);
 
@@ -301,7 +306,7 @@ int scft_batch_tuning(const scft_batch *b, int *n_buckets, int *bucket_nmax,
  * (n unknowns) in; d_phi (n, nullable), d_r = phi - phi_t (n), d_rnorm
  * (1 double) and d_status (1 word, SCFT_ST_* bits) out.  Walls at w = 0, the
  * implicit-Euler stepper, the march variant of a one-instance batch (so the
- * same bits as scft_batch_eval).  Calls no allocating routine: the working
+ * same bits as scft_batch_eval of one).  Calls no allocating routine: the working
  * memory (descriptor, pairing weights, work counter, q-slabs) is a fixed
  * device array of 64 MiB + 256 KiB per GPU that the library holds until the
  * process ends.  The slabs need (N/2) * cap * 8 bytes, cap = the power of

@@ -583,8 +583,8 @@ extern "C" int scft_batch_create(scft_batch** out, const scft_batch_desc* dsc) {
   b->uoff.resize(b->n_inst);
   for (int k = 0; k < b->n_inst; k++) {
     const int M = dsc->M[k], N = dsc->N[k];
-    // N: a power of two (Romberg) in [16, 16384] (the N/2 + 1 pairing weights
-    // of a bucket are held in LDS)
+    // N: a power of two (Romberg) in [16, 16384] (IRK4 holds the N/2 + 1 pairing
+    // weights of a bucket in LDS; a workgroup's slabs stay within a 32-bit offset)
     // up to 4096 unknowns (both steppers)
     const int n_max = 4096;
     if (M < 3 || (b->bc == SCFT_BC_DD ? M - 2 : M - 1) > n_max || N < 16 || N > 16384 ||

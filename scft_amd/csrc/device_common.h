@@ -208,12 +208,6 @@ __device__ __forceinline__ dd dd_mul(dd a, dd b) {
   return quick_two_sum(p.h, p.l);
 }
 __device__ __forceinline__ dd dd_scale(dd a, double s) { return {a.h * s, a.l * s}; }  // s = 2^k
-__device__ __forceinline__ double dd_div_to_double(dd a, dd b) {
-#pragma clang fp contract(off)
-  const double q1 = a.h / b.h;
-  const dd r = dd_add(a, dd_mul(b, dd_from(-q1)));
-  return q1 + r.h / b.h;
-}
 
 // 2x2 double-double product R = X * Y, rescaled by a power of two so the
 // largest entry is in [1, 2): the pivot is a ratio of entries, so scaling is

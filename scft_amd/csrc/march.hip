@@ -47,10 +47,13 @@
 //     whatever the variant (640 G node-steps/s), and at that traffic the clock
 //     falls to 1.6 GHz.  With every fourth slab and 1.375 N steps the vector
 //     units bound it (72% busy at 1.9 GHz): 970-1120 G node-steps/s.
-//   * accuracy: the rows of G are computed in double-double and every weight
-//     is positive, so nothing cancels: phi is 10-100 times closer to an
-//     extended-precision march than with pivots rounded to double (m = 4095,
-//     N = 4096, uniform: 5e-14 against 1.4e-11).
+//   * accuracy: the rows of G are computed in double-double and rounded once.
+//     Where neighbours couple negatively (dt > h^2 / 6) every weight is positive
+//     and nothing cancels; where they do not, f and h are negative, but below
+//     0.27 in size on a uniform mesh, so a row reaches a few neighbours only.
+//     phi against an extended-precision march, uniform, m = 4095: 1.1e-14 for
+//     N = 128, 5e-14 for N = 4096 (2.9e-13 and 2.1e-12 with pivots rounded to
+//     double).
 // No MFMA: nothing here is a dense contraction.
 #include "scft_internal.h"
 #include "device_common.h"
@@ -417,9 +420,10 @@ __device__ void march_one(const MarchArgs& a, const int inst, const unsigned st0
     }
     // Second half, segment by segment: the slabs g SEG .. g SEG + SEG - 1 into
     // this lane's own places in LDS (the kept one, loaded a segment ahead,
-    // then SEG - 1 steps from it: the same operations as in the first half, so
-    // the same bits), then SEG steps of the march that pair with them from the
-    // top down.
+    // then SEG - 1 steps from it: those of the first half to rounding, since a
+    // lane's two outer neighbours are read from the lanes beside it here and
+    // come out of its own inflows there), then SEG steps of the march that pair
+    // with them from the top down.
     auto lds_slot = [&](const int e) __attribute__((always_inline)) {
       return seg_lds + e * (P * K) + (K >= 2 ? 2 * tid : tid);
     };
