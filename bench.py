@@ -37,8 +37,9 @@ Also reported:
                 evaluation sweep: algorithmic bytes (the q-slabs it keeps, written
                 and read back, O(n) I/O) over its HIP-event duration, against
                 8 TB/s.  A batch that fills the chip keeps every fourth slab
-                and recomputes the others, so that HBM no longer bounds it but
-                the FP64 vector units do
+                and recomputes the others: `bound` is then "fp64" (the vector
+                units), the GB/s are what is left of the traffic, and
+                gnodesteps_per_s is the rate of the march
   cpu_baseline  the CPU oracle (same mixer, same tolerance, cold start) on a
                 bounded sample of the same instances, threads over the host
                 cores the GPU box allots to one GPU; beside it the reference
@@ -194,6 +195,20 @@ def march_source_sha256():
         with open(os.path.join(ROOT, "scft_amd", "csrc", name), "rb") as f:
             h.update(f.read())
     return h.hexdigest()
+
+
+def kept_bytes(cfg, buckets, tuning):
+    """Algorithmic bytes of one evaluation of each instance (the q-slabs that
+    its launch keeps, written and read back, and O(n) I/O), whether its launch
+    recomputes slabs, and its bucket: from the bytes that each bucket's launch
+    reports, every slab's or every fourth's."""
+    n = np.array([len(x) - 1 for x in cfg["xs"]])
+    N = np.array(cfg["Ns"])
+    every, fourth = 8.0 * n * (N - 2) + 40.0 * n, 8.0 * n * 2 * (N // 8) + 40.0 * n
+    bucket = np.searchsorted([t[0] for t in tuning], n)  # n_max, ascending
+    recomputes = np.array([abs(fourth[bucket == i].sum() - by) < abs(every[bucket == i].sum() - by)
+                           for i, (_, _, by) in enumerate(buckets)])[bucket]
+    return np.where(recomputes, fourth, every), recomputes, bucket
 
 
 def measured_traffic(workload, kern, n_items, alg_bytes):
@@ -677,6 +692,9 @@ def main():
     n_items, ms, by = buckets[di]
     kern = f"march_kernel<{tuning[di][1]}, {tuning[di][2]}>"
     achieved = by / (ms * 1e-3) / 1e9
+    by_instance, recomputes, bucket = kept_bytes(cfg, buckets, tuning)
+    steps = sum((len(cfg["xs"][k]) - 1.0) * cfg["Ns"][k] for k in np.flatnonzero(bucket == di))
+    bound = "fp64" if recomputes[bucket == di].all() else "hbm"
     sweep_ms = sum(t[1] for t in buckets)
     log(f"bench: buckets (items, ms, GB) = {[(i, round(m, 3), round(bb / 1e9, 3)) for i, m, bb in buckets]}")
     log(f"bench: one sweep {sweep_ms:.2f} ms, dominant launch {ms:.3f} ms, {achieved:.1f} GB/s")
@@ -713,7 +731,7 @@ def main():
     res = warm["res"] if warm else res_cold
     total = warm["total"] if warm else total_cold
     value = warm["value"] if warm else value_cold
-    gb_eff = res["bytes"] / (total / args.steps) / 1e9
+    gb_eff = float(np.dot(res["iters"], by_instance)) / (total / args.steps) / 1e9
 
     out = {
         "metric": METRIC,
@@ -746,11 +764,12 @@ def main():
             },
         },
         "roofline": {
-            "bound": "hbm",
+            "bound": bound,
             "achieved": round(achieved, 1),
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
+            "gnodesteps_per_s": round(steps / ms / 1e6, 1),
             "traffic": measured_traffic(args.workload, kern, n_items, by),
             "kernel": f"{kern}: bucket of {n_items} instances, {ms:.3f} ms per launch",
         },
