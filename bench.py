@@ -42,7 +42,7 @@ Also reported:
                 gnodesteps_per_s is the rate of the march
   cpu_baseline  the CPU oracle (same mixer, same tolerance, cold start) on a
                 bounded sample of the same instances, threads over the host
-                cores the GPU box allots to one GPU; beside it the reference
+                cores that OMP_NUM_THREADS allots; beside it the reference
                 problem of configuration 1 (m = 32, N = 2048, w0 = 0, plain
                 Anderson, history 10, mixing 0.1) solved single-threaded
 """
@@ -780,8 +780,7 @@ def main():
     out["config"]["audit"] = audit(S, cfg, b, res)
     log(f"bench: audit {out['config']['audit']}")
     if not args.no_cpu and res_cold is not None:
-        # the host cores the GPU box allots to one GPU (OMP_NUM_THREADS there;
-        # the whole host may show more): every one of them
+        # every host core that OMP_NUM_THREADS allots (the whole host may show more)
         affinity = len(os.sched_getaffinity(0))
         threads = int(os.environ.get("OMP_NUM_THREADS", "0") or 0) or affinity
         threads = max(1, min(threads, affinity))

@@ -1,8 +1,8 @@
 """ctypes front end of the CPU oracle (oracle/liboracle.so).
 
 TEST INFRASTRUCTURE ONLY: imported by tests/, by __graft_entry__.smoke() and
-by bench.py's CPU-baseline leg, always as the checker.  The product library
-(scft_amd/) never imports it.
+by bench.py's CPU-baseline leg, always as what results are compared with.  The
+product library (scft_amd/) never imports it.
 
 The C sources cite the reference lines they restate; this module only
 marshals numpy arrays.  `ref` gives access to the reference's own

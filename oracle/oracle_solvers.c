@@ -5,7 +5,7 @@
  * helpers), plus the safeguarded residual-form Anderson mixer that the
  * batched device solver implements.
  *
- * TEST INFRASTRUCTURE ONLY (the checker); arrays here are 0-based, the
+ * TEST INFRASTRUCTURE ONLY; arrays here are 0-based, the
  * reference's are 1-based Numerical-Recipes offsets.
  */
 #include "oracle_solvers.h"

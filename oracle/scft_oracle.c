@@ -1,7 +1,7 @@
 /*
  * scft_oracle.c -- CPU restatement of giantsda/SCFT's inner field evaluation.
  *
- * TEST INFRASTRUCTURE ONLY (the checker): used by tests/, by the smoke check
+ * TEST INFRASTRUCTURE ONLY: used by tests/, by the smoke check
  * and by bench.py's CPU-baseline leg; never by the product library.
  *
  * Each function cites the reference lines it restates.  "Mode R" is the

@@ -3,7 +3,7 @@
  *
  * TEST INFRASTRUCTURE ONLY.  Nothing in the product library links or calls
  * this code; only tests/, __graft_entry__.smoke() and bench.py's CPU-baseline
- * leg use it, and only as the checker.
+ * leg use it, and only to compare with.
  *
  * Conventions (all FP64):
  *   M      number of mesh nodes (m = M-1 linear elements)
