@@ -1,5 +1,5 @@
-"""What the plan of a batch's sweep promises beyond its results: scratch, the
-slab regime, and launches that do not wait for each other without need."""
+"""What the plan of a batch's sweep promises beyond its results: its scratch and
+the slabs it keeps."""
 import ctypes as C
 
 import numpy as np
